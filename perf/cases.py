@@ -164,9 +164,11 @@ def work(case):
 
 
 def tolerance(case):
-    """Outputs are bf16. A decode rounds once: a relative 2-norm of 1.7e-3 against 64 bits.
-    A prefill's readout products take bf16 operands too: 2.9e-3."""
-    return {"rel": 6e-3, "max": 0.03} if case["kind"] == "decode" else {"rel": 1.2e-2, "max": 0.1}
+    """Outputs are bf16. A decode rounds once: a relative 2-norm of 1.7e-3 against 64 bits, at
+    most 3.9e-3 of an element.
+    A prefill's readout products take bf16 operands too: 2.9e-3, at most
+    4.6e-2 of the root mean square."""
+    return {"rel": 6e-3, "max": 0.016} if case["kind"] == "decode" else {"rel": 1.2e-2, "max": 0.2}
 
 
 def exact(case, seed):
