@@ -25,11 +25,12 @@
 //         fp32-valued operands on the state path (S0, R, T, U) are split into bf16
 //         hi + lo halves so the state keeps ~2^-16 relative accuracy. With few
 //         sequences, long ones are cut into segments scanned in parallel (two scan
-//         launches over job tables).
+//         launches over job tables). With many sequences the scan runs on 32x32 tiles,
+//         32 state rows per wave and two workgroups per CU (gdn_prefill_wide.hip).
 //
 // Files: gdn_prefill.h (records, layouts, argument structs, shared helpers),
-// gdn_prefill_plan.hip, gdn_prefill_prep.hip, gdn_prefill_scan.hip (the kernels) and
-// gdn_prefill.hip (workspace layout and launches behind gdn_prefill_launch).
+// gdn_prefill_plan.hip, gdn_prefill_prep.hip, gdn_prefill_scan.hip, gdn_prefill_wide.hip (the
+// kernels) and gdn_prefill.hip (workspace layout and launches behind gdn_prefill_launch).
 #pragma once
 
 #include "gdn_common.h"
@@ -454,6 +455,63 @@ struct ScanArgs {
 };
 
 
+// A scan workgroup's job: its (sequence or segment job, q/k head) group grp, its place wi
+// among the group's workgroups, and the job's sequence, kind and chunk range.
+struct ScanJob {
+    int grp, wi, n, tok0, len, c0, kind, cb, ce, q, steps, last;
+};
+
+// Finds this workgroup's job (SEG: in the segment job table); false when it has none.
+template <int NW, bool SEG>
+__device__ __forceinline__ bool scan_job(const ScanArgs &p, ScanJob &j)
+{
+    constexpr int TPH = 8 / NW;  // workgroups per (sequence, v-head)
+    // Workgroups of one (sequence, q/k head) share K, Q through L2: one XCD for them all
+    // (workgroup ids are dealt to the 8 XCDs round-robin).
+    const int pid = blockIdx.x, xcd = pid & 7, slot = pid >> 3;
+    const int gsz = TPH * p.ratio;
+    j.wi = slot % gsz;
+    j.grp = (slot / gsz) * 8 + xcd;
+    if (j.grp >= p.ngroups)
+        return false;
+    j.kind = kJobFirst;
+    j.cb = 0;
+    j.ce = 0x7fffffff;
+    j.q = -1;
+    j.steps = 0;
+    j.last = 0;
+    if constexpr (SEG) {
+        // the grid covers the job table's capacity, so the entry exists even past the job
+        // count, and both load together
+        const int e = j.grp / p.HQK;
+        const int4 *je = (const int4 *)(p.jobs + kJobInts * (p.job_first + e));
+        const int4 j0 = je[0], j1 = je[1], j2 = je[2];
+        if (e >= p.header[p.njob_idx])
+            return false;
+        j.n = j0.x;
+        j.kind = j0.y;
+        j.cb = j0.z;
+        j.ce = j0.w;
+        j.q = j1.x;
+        j.steps = j1.y;
+        j.last = j1.z;
+        j.tok0 = j1.w;
+        j.len = j2.x;
+        j.c0 = j2.y;
+    } else {
+        // ranks below ngroups / HQK = N all have an entry: load it with the count
+        const int e = j.grp / p.HQK;
+        const int4 r = *(const int4 *)(p.seq_rank + 4 * e);
+        if (p.njob_idx > 0 && e >= p.header[p.njob_idx])
+            return false;
+        j.n = r.x;
+        j.tok0 = r.y;
+        j.len = r.z;
+        j.c0 = r.w;
+    }
+    return true;
+}
+
 // LDS layouts (16-byte units). A ds_read_b128 is served in four cycles of 16 lanes: the
 // lanes of one 32-lane half whose lane bits 2, 3, 4 have equal parity; a cycle is
 // conflict-free when its 16 lanes touch 16 distinct units modulo 256 bytes (measured on
@@ -532,8 +590,8 @@ struct ScanBuf {
 };
 
 // ------------------------------------------------------------------------- kernels
-// Defined in gdn_prefill_plan.hip, gdn_prefill_prep.hip and gdn_prefill_scan.hip; the
-// scan kernels are instantiated there for SEG = false (whole sequences) and true
+// Defined in gdn_prefill_plan.hip, gdn_prefill_prep.hip, gdn_prefill_scan.hip and
+// gdn_prefill_wide.hip; the scan4 / scan8 kernels are instantiated there for SEG = false (whole sequences) and true
 // (segment jobs).
 __global__ __launch_bounds__(256) void gdn_prefill_plan_kernel(PlanArgs p);
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void
@@ -544,5 +602,7 @@ template <bool SEG>
 __global__ __launch_bounds__(512) void gdn_prefill_scan8_kernel(ScanArgs p);
 template <bool SEG>
 __global__ __launch_bounds__(256) void gdn_prefill_scan4_kernel(ScanArgs p);
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+gdn_prefill_scanw_kernel(ScanArgs p);
 
 }  // namespace gdn

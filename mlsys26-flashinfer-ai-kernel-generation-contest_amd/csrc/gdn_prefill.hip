@@ -238,6 +238,16 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
     // their LDS). Above 256 pairs the 8-wave scan alone (the 4-wave one rarely wins there).
     const bool whole_dual = G == 1 && p->variant == 0 && self_plan && (int64_t)N * HV > 128 &&
                             (int64_t)N * HV <= 256;
+    // With three (sequence, v-head) pairs per CU and more, of at most six chunks on average, a
+    // pair's start and end (state and first chunk in, state out) weigh as much as its chunks:
+    // the wide scan, whose two workgroups per CU cover one another's. Measured on MI355X, 8-wave
+    // against wide scan, whole prefill: 100 sequences of 1 to 130 tokens at 32 v-heads 205 ->
+    // 181 us, 64 of 128 162 -> 145, 40 of 64 to 200 108 -> 100, 24 of 1 to 100 56 -> 51, 100 of
+    // 64 to 256 at 8 v-heads 97 -> 91. Fewer pairs gain nothing (20 of 300 to 500 at 32 v-heads
+    // 114.5 -> 115.5, 16 of 64 to 1024 124 -> 128: two long jobs share a CU's time), nor do
+    // longer sequences (32 of 512 209 -> 212, 64 of 1000 728 -> 743).
+    const bool wide = G == 1 && p->variant == 0 && (int64_t)N * HV >= 3 * (int64_t)num_cus(st) &&
+                      T <= 384 * (int64_t)N;
     pa.whole_cus = whole_dual ? num_cus(st) : 0;
     gdn_begin_launches();
     int rc = 0;
@@ -334,7 +344,7 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
         // 8 waves per workgroup = one (sequence, v-head) each, two waves per SIMD; with
         // few (sequence, v-head) pairs, 4 waves and two workgroups per pair spread the
         // state rows over twice as many CUs. variant: 1 forces 4 waves, 2 forces 8.
-        auto scan = [&](int64_t units, bool nw4) {
+        auto scan = [&](int64_t units, bool nw4, bool wide = false) {
             const int64_t ngroups = units * HQK;
             sa.ngroups = (int)ngroups;
             const int tph = nw4 ? 2 : 1;
@@ -342,7 +352,9 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
             if (ngroups > 0x7fffffff || blocks > 0x7fffffff)
                 return gdn_set_error(GDN_EINVAL, "gdn_prefill: grid too large");
             const dim3 grid((unsigned)blocks), b4(256), b8(512);
-            if (sa.jobs && nw4)
+            if (wide)
+                hipLaunchKernelGGL(gdn::gdn_prefill_scanw_kernel, grid, b4, 0, st, sa);
+            else if (sa.jobs && nw4)
                 hipLaunchKernelGGL(gdn::gdn_prefill_scan4_kernel<true>, grid, b4, 0, st, sa);
             else if (sa.jobs)
                 hipLaunchKernelGGL(gdn::gdn_prefill_scan8_kernel<true>, grid, b8, 0, st, sa);
@@ -377,7 +389,7 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
                 rc = scan(N, false);
             }
         } else {
-            rc = scan(N, nw4);
+            rc = scan(N, nw4, wide);
         }
         if (rc)
             return rc;

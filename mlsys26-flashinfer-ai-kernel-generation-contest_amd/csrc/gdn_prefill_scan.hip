@@ -25,63 +25,6 @@ namespace gdn {
 // V columns are read with the LDS transpose read.
 // SEG: the grid walks segment jobs (p.jobs); otherwise whole sequences, and none of the
 // segment code is compiled in (it costs the whole-sequence loop registers).
-// A scan workgroup's job: its (sequence or segment job, q/k head) group grp, its place wi
-// among the group's workgroups, and the job's sequence, kind and chunk range.
-struct ScanJob {
-    int grp, wi, n, tok0, len, c0, kind, cb, ce, q, steps, last;
-};
-
-// Finds this workgroup's job (SEG: in the segment job table); false when it has none.
-template <int NW, bool SEG>
-__device__ __forceinline__ bool scan_job(const ScanArgs &p, ScanJob &j)
-{
-    constexpr int TPH = 8 / NW;  // workgroups per (sequence, v-head)
-    // Workgroups of one (sequence, q/k head) share K, Q through L2: one XCD for them all
-    // (workgroup ids are dealt to the 8 XCDs round-robin).
-    const int pid = blockIdx.x, xcd = pid & 7, slot = pid >> 3;
-    const int gsz = TPH * p.ratio;
-    j.wi = slot % gsz;
-    j.grp = (slot / gsz) * 8 + xcd;
-    if (j.grp >= p.ngroups)
-        return false;
-    j.kind = kJobFirst;
-    j.cb = 0;
-    j.ce = 0x7fffffff;
-    j.q = -1;
-    j.steps = 0;
-    j.last = 0;
-    if constexpr (SEG) {
-        // the grid covers the job table's capacity, so the entry exists even past the job
-        // count, and both load together
-        const int e = j.grp / p.HQK;
-        const int4 *je = (const int4 *)(p.jobs + kJobInts * (p.job_first + e));
-        const int4 j0 = je[0], j1 = je[1], j2 = je[2];
-        if (e >= p.header[p.njob_idx])
-            return false;
-        j.n = j0.x;
-        j.kind = j0.y;
-        j.cb = j0.z;
-        j.ce = j0.w;
-        j.q = j1.x;
-        j.steps = j1.y;
-        j.last = j1.z;
-        j.tok0 = j1.w;
-        j.len = j2.x;
-        j.c0 = j2.y;
-    } else {
-        // ranks below ngroups / HQK = N all have an entry: load it with the count
-        const int e = j.grp / p.HQK;
-        const int4 r = *(const int4 *)(p.seq_rank + 4 * e);
-        if (p.njob_idx > 0 && e >= p.header[p.njob_idx])
-            return false;
-        j.n = r.x;
-        j.tok0 = r.y;
-        j.len = r.z;
-        j.c0 = r.w;
-    }
-    return true;
-}
-
 // SEG: the body handles every segment job kind; otherwise only jobs from the initial state
 // with outputs into new_state (whole sequences), with none of the segment code compiled in.
 // OUTS (segment bodies): 1 compiles the body for jobs with outputs (kJobFirst, kJobResume),

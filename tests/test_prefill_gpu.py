@@ -297,6 +297,20 @@ def test_prefill_many_sequences(dev, nseq):
     _run(dev, prefill_inputs(lens, hqk=4, hv=8, seed=nseq, with_state=True), f"N={nseq}")
 
 
+@pytest.mark.parametrize("lens,hqk,hv,state,gates", [
+    # the scan with two workgroups per CU (768 (sequence, v-head) pairs and more): chunk edges
+    # and remainders, empty sequences, odd and even chunk counts, the smallest batch it takes
+    ([1, 63, 64, 65, 0, 127, 128, 129, 191, 192, 193, 257, 31, 2, 320, 16, 17, 96, 64, 33, 5, 48,
+      80, 15], 16, 32, True, "mild"),
+    ([64] * 24, 16, 32, False, "strong"),
+    ([7 + 3 * i for i in range(96)], 4, 8, True, "none"),
+    ([40, 0, 130] * 43, 2, 6, True, "mild"),
+])
+def test_prefill_wide_scan(dev, lens, hqk, hv, state, gates):
+    _run(dev, prefill_inputs(lens, hqk=hqk, hv=hv, seed=sum(lens) % 97, with_state=state,
+                             gates=gates), f"wide scan {len(lens)} x {hv}")
+
+
 @pytest.mark.parametrize("nseq", [3, 64, 300])
 def test_prefill_gap_before_first_sequence(dev, nseq):
     """cu_seqlens[0] > 0: the leading tokens belong to no sequence and read as zero."""
