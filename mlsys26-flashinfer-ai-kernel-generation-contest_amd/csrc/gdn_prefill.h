@@ -601,7 +601,7 @@ gdn_prefill_prep2_kernel(PrepArgs p);
 template <bool SEG>
 __global__ __launch_bounds__(512) void gdn_prefill_scan8_kernel(ScanArgs p);
 template <bool SEG>
-__global__ __launch_bounds__(256) void gdn_prefill_scan4_kernel(ScanArgs p);
+__global__ __launch_bounds__(320) void gdn_prefill_scan4_kernel(ScanArgs p);
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 gdn_prefill_scanw_kernel(ScanArgs p);
 

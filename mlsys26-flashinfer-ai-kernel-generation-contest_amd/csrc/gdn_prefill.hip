@@ -351,9 +351,10 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
             const int64_t blocks = 8 * ((int64_t)tph * ratio) * ((ngroups + 7) / 8);
             if (ngroups > 0x7fffffff || blocks > 0x7fffffff)
                 return gdn_set_error(GDN_EINVAL, "gdn_prefill: grid too large");
-            const dim3 grid((unsigned)blocks), b4(256), b8(512);
+            // (scan4: four compute waves and the copy wave)
+            const dim3 grid((unsigned)blocks), bw(256), b4(320), b8(512);
             if (wide)
-                hipLaunchKernelGGL(gdn::gdn_prefill_scanw_kernel, grid, b4, 0, st, sa);
+                hipLaunchKernelGGL(gdn::gdn_prefill_scanw_kernel, grid, bw, 0, st, sa);
             else if (sa.jobs && nw4)
                 hipLaunchKernelGGL(gdn::gdn_prefill_scan4_kernel<true>, grid, b4, 0, st, sa);
             else if (sa.jobs)

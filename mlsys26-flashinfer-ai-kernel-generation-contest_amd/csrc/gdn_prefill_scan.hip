@@ -2,6 +2,8 @@
 // sequences or segment jobs.
 #include "gdn_prefill.h"
 
+#include <cstddef>
+
 namespace gdn {
 
 // Copy windows of one chunk, 64 units (1 KB) each: K rows 4b..4b+3 (16 windows), Q (16),
@@ -90,42 +92,45 @@ __device__ __forceinline__ void scan_body(const ScanArgs &p, const ScanJob &job,
     constexpr int VWIN = 2 * NW;               // V windows
     constexpr int NWIN = 32 + VWIN + 19;       // all windows
     constexpr int PER = (NWIN + NW - 1) / NW;  // windows per wave
+    // The 4-wave scan's copies are issued by a fifth wave. One compute wave per SIMD issues
+    // alone, and its 17 copies a chunk cost it 0.5-0.6k of 5.1k cycles (measured by leaving them
+    // out: the four waves' copies meet at the CU's one address unit). Whole prefills with the
+    // copy wave, bit-identical: 1 x 300 at 32 v-heads 21.8 -> 20.0 us, 1 x 1024 at 8 v-heads
+    // 36.6 -> 32.4, 8 sequences of 64 to 1024 at 8 v-heads 44.0 -> 39.9. The 8-wave scan has half
+    // the copies per wave and a second wave per SIMD to cover them: a ninth wave there cost
+    // 1-2 % (12 of 600 at 32 v-heads 106 -> 109 us).
+    constexpr bool kCopier = NW == 4;
 
-    // Source offset of this lane in window i (compile-time) of this wave; window kinds
-    // follow win = w + NW i: K rows 4b..4b+3 (16 windows), Q (16), V (NW == 8: 4 rows per
-    // window, NW == 4: 8 rows), then 18 T' / P' windows and the gate area.
-    uint32_t woff[PER];
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const int win = w + NW * i;
-        uint32_t off = 0;
-        if (NW * i < 16) {
+    // Source offset of this lane in a window; windows are K rows 4b..4b+3 (16 windows), Q (16),
+    // V (NW == 8: 4 rows per window, NW == 4: 8 rows), then 18 T' / P' windows and the gate
+    // area. first: the lowest window of win's group of waves, which decides the kind.
+    auto win_off = [&](int first, int win) -> uint32_t {
+        if (first < 16) {
             const int t = 4 * win + (l >> 4), cs = l & 15;
-            off = (uint32_t)t * kst2 + 16u * (cs ^ kswz(t));
-        } else if (NW * i < 32) {
+            return (uint32_t)t * kst2 + 16u * (cs ^ kswz(t));
+        }
+        if (first < 32) {
             const int t = 4 * (win - 16) + (l >> 4), cs = l & 15;
-            off = (uint32_t)t * qst2 + 16u * (cs ^ (t & 15));
-        } else if (NW * i < 32 + VWIN) {
+            return (uint32_t)t * qst2 + 16u * (cs ^ (t & 15));
+        }
+        if (first < 32 + VWIN) {
             const int b = win - 32;
             const int t = NW == 8 ? 4 * b + (l >> 4) : 8 * b + (l >> 3);
             const int cs = NW == 8 ? (l & 15) : (l & 7);
-            off = (uint32_t)t * vst2 + 16u * (cs ^ (2 * (t & 3)));
-        } else {
-            const int r = win - 32 - VWIN;
-            if (r < 18) {
-                const int mt = r / 6, pr = r % 6, b = pr == 0 ? 0 : (pr == 1 ? 2 : pr + 2);
-                const int u = 64 * b + l;  // this lane's LDS unit
-                const int row = mt < 2 ? tlay_row(u) : play_row(u), cc = lay_col(u);
-                const int bi = row >> 4, bj = cc >> 1;
-                const int mbase = mt == 0 ? kRecThi : (mt == 1 ? kRecTlo : kRecP);
-                off = bj <= bi ? (uint32_t)(mbase + (tri_blk(bi, bj) * 32 + 2 * (row & 15) + (cc & 1)) * 16)
-                               : (uint32_t)kRecZero;
-            } else {
-                off = kRecGates + 16u * l;
-            }
+            return (uint32_t)t * vst2 + 16u * (cs ^ (2 * (t & 3)));
         }
-        woff[i] = off;
-    }
+        const int r = win - 32 - VWIN;
+        if (r < 18) {
+            const int mt = r / 6, pr = r % 6, b = pr == 0 ? 0 : (pr == 1 ? 2 : pr + 2);
+            const int u = 64 * b + l;  // this lane's LDS unit
+            const int row = mt < 2 ? tlay_row(u) : play_row(u), cc = lay_col(u);
+            const int bi = row >> 4, bj = cc >> 1;
+            const int mbase = mt == 0 ? kRecThi : (mt == 1 ? kRecTlo : kRecP);
+            return bj <= bi ? (uint32_t)(mbase + (tri_blk(bi, bj) * 32 + 2 * (row & 15) + (cc & 1)) * 16)
+                            : (uint32_t)kRecZero;
+        }
+        return kRecGates + 16u * l;
+    };
 
     // Buffer ranges of chunk c: K / Q / V end after the chunk's last row.
     struct ChunkSrc {
@@ -144,19 +149,17 @@ __device__ __forceinline__ void scan_body(const ScanArgs &p, const ScanJob &job,
         cs.r = __builtin_amdgcn_make_buffer_rsrc((void *)(rbase + c * rstep), 0, valid ? kRecBytes : 0, 0x00020000);
         return cs;
     };
-    auto chunk_src = [&](int c) { return chunk_src_v(c, true); };
-    auto issue_win = [&](ScanBuf<NW> &B, const ChunkSrc &cs, const int i) {
-        const int win = w + NW * i;  // window kind is a compile-time function of i
-        if (NW * i < 16) {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(cs.k, (GDN_LDS void *)&B.K[64 * win], 16, woff[i], 0, 0, 0);
-        } else if (NW * i < 32) {
+    auto issue_win = [&](ScanBuf<NW> &B, const ChunkSrc &cs, int first, int win, uint32_t off) {
+        if (first < 16) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(cs.k, (GDN_LDS void *)&B.K[64 * win], 16, off, 0, 0, 0);
+        } else if (first < 32) {
             if (OUTS == 0 || OUTS == 2)  // state maps read neither Q nor P'
                 return;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(cs.q, (GDN_LDS void *)&B.Q[64 * (win - 16)], 16, woff[i], 0, 0, 0);
-        } else if (NW * i < 32 + VWIN) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(cs.q, (GDN_LDS void *)&B.Q[64 * (win - 16)], 16, off, 0, 0, 0);
+        } else if (first < 32 + VWIN) {
             if (OUTS == 2)  // identity rows: V = 0
                 return;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(cs.v, (GDN_LDS void *)&B.V[64 * (win - 32)], 16, woff[i], 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(cs.v, (GDN_LDS void *)&B.V[64 * (win - 32)], 16, off, 0, 0, 0);
         } else if (win < NWIN) {
             const int r = win - 32 - VWIN;
             if (r < 18) {
@@ -164,17 +167,91 @@ __device__ __forceinline__ void scan_body(const ScanArgs &p, const ScanJob &job,
                 if ((OUTS == 0 || OUTS == 2) && mt == 2)
                     return;
                 u32x4 *dst = mt == 2 ? &B.P[64 * b] : &B.T[mt][64 * b];
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(cs.r, (GDN_LDS void *)dst, 16, woff[i], 0, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(cs.r, (GDN_LDS void *)dst, 16, off, 0, 0, 0);
             } else {
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(cs.r, (GDN_LDS void *)&B.G[0], 16, woff[i], 0, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(cs.r, (GDN_LDS void *)&B.G[0], 16, off, 0, 0, 0);
             }
         }
     };
-    auto issue_chunk = [&](ScanBuf<NW> &B, int c) {
-        const ChunkSrc cs = chunk_src(c);
+
+    // ---- the copy wave of the 4-wave scan (wave 4): every window of every chunk. It waits for
+    // its copies and meets the compute waves at the barrier before each chunk (and at those of
+    // the chain steps, which precede the loop and do not touch BA).
+    if constexpr (kCopier) {
+        if (w == NW) {
+            // K window b: rows 4 b + r, r = l / 16, whose swizzle is kswz(r) ^ kswz(4 b) (Q:
+            // r ^ 4 (b % 4)); V window b: rows 8 b + l / 8, the same swizzle for every b. One
+            // register per matrix, re-derived per chunk so that the windows' offsets are not
+            // all kept, and one per record window.
+            const int r = l >> 4, cs = l & 15;
+            uint32_t rk = r * kst2, rq = r * qst2, sk4 = 16u * (cs ^ kswz(r)), sq4 = 16u * (cs ^ r),
+                     rv = win_off(32, 32), rr[19];
+#pragma unroll
+            for (int i = 0; i < 19; ++i)
+                rr[i] = win_off(32 + VWIN + i, 32 + VWIN + i);
+            // (destinations as LDS byte addresses: the two buffers' copies may be merged into
+            // one piece of code, whose selected pointer must not become a generic one)
+            typedef ScanBuf<NW> Buf;
+            const uint32_t la = (uint32_t)(uintptr_t)(GDN_LDS char *)&BA,
+                           lb = (uint32_t)(uintptr_t)(GDN_LDS char *)&BB;
+            auto issue = [&](uint32_t buf, int c) {
+                const ChunkSrc src = chunk_src_v(c, true);
+                asm volatile("" : "+v"(rk), "+v"(rq), "+v"(sk4), "+v"(sq4), "+v"(rv));
+                auto copy = [&](__amdgpu_buffer_rsrc_t rs, uint32_t dst, uint32_t off) {
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (GDN_LDS void *)(uintptr_t)(buf + dst), 16, off, 0, 0, 0);
+                };
+#pragma unroll
+                for (int b = 0; b < 16; ++b)
+                    copy(src.k, offsetof(Buf, K) + 1024 * b, rk + 4 * b * kst2 + (sk4 ^ (16u * kswz(4 * b))));
+                if (OUTS != 2)  // identity rows: V = 0
+#pragma unroll
+                    for (int b = 0; b < VWIN; ++b)
+                        copy(src.v, offsetof(Buf, V) + 1024 * b, rv + 8 * b * vst2);
+#pragma unroll
+                for (int i = 0; i < 19; ++i) {
+                    const int mt = i / 6, pr = i % 6, b = pr == 0 ? 0 : (pr == 1 ? 2 : pr + 2);
+                    if ((OUTS == 0 || OUTS == 2) && mt == 2)  // state maps read neither Q nor P'
+                        continue;
+                    copy(src.r, (i == 18 ? offsetof(Buf, G) : mt == 2 ? offsetof(Buf, P) : offsetof(Buf, T) + 8192 * mt) +
+                                    (i == 18 ? 0 : 1024 * b), rr[i]);
+                }
+                if (OUTS != 0 && OUTS != 2)
+#pragma unroll
+                    for (int b = 0; b < 16; ++b)
+                        copy(src.q, offsetof(Buf, Q) + 1024 * b, rq + 4 * b * qst2 + (sq4 ^ (64u * (b & 3))));
+            };
+            if (ce > cb)
+                issue(la, cb);
+            for (int m = 0; m < steps; ++m) {
+                __builtin_amdgcn_s_barrier();
+                if (m + 1 < steps)
+                    __builtin_amdgcn_s_barrier();
+            }
+            for (int c = cb; c < ce; c += 2) {
+                dma_barrier();
+                if (c + 1 >= ce)
+                    break;
+                issue(lb, c + 1);
+                dma_barrier();
+                if (c + 2 < ce)
+                    issue(la, c + 2);
+            }
+            return;
+        }
+    }
+
+    uint32_t woff[PER];
+    if constexpr (!kCopier) {
 #pragma unroll
         for (int i = 0; i < PER; ++i)
-            issue_win(B, cs, i);
+            woff[i] = win_off(NW * i, w + NW * i);
+    }
+    auto issue_chunk = [&](ScanBuf<NW> &B, const ChunkSrc &cs) {
+        if constexpr (!kCopier) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+                issue_win(B, cs, NW * i, w + NW * i, woff[i]);
+        }
     };
     // ---- LDS read offsets (bytes within a ScanBuf member; chunk-invariant)
     const int c_ = lr & 3, r_ = lr >> 2;
@@ -222,12 +299,9 @@ __device__ __forceinline__ void scan_body(const ScanArgs &p, const ScanJob &job,
         issue_m(q);
         load_r(q);
         // unconditional, so the number of operations in flight is the same on every path
-        const ChunkSrc cs = chunk_src_v(cb, ce > cb);
-#pragma unroll
-        for (int i = 0; i < PER; ++i)
-            issue_win(BA, cs, i);
+        issue_chunk(BA, chunk_src_v(cb, ce > cb));
     } else if (ce > cb) {
-        issue_chunk(BA, cb);
+        issue_chunk(BA, chunk_src_v(cb, true));
     }
 
     // ---- state: S[2 s + h] holds S[v0w + lr][32 s + 8 lg + 4 h + i], i = 0..3
@@ -262,7 +336,7 @@ __device__ __forceinline__ void scan_body(const ScanArgs &p, const ScanJob &job,
     // LDS unit 16 j + (cu ^ kswz(j)) holds row j, k-chunk cu (the K layout of the loop).
     if (chain) {
         for (int m = 0; m < steps; ++m) {
-            if (m == 0) {
+            if (m == 0 && !kCopier) {
                 // M_q^T and R_q are in (memory operations complete in order); the first
                 // chunk's copies, at least NWIN / NW per wave, may still be in flight
                 constexpr int nv = NWIN / NW;
@@ -329,8 +403,8 @@ __device__ __forceinline__ void scan_body(const ScanArgs &p, const ScanJob &job,
     auto issue_slot = [&](ScanBuf<NW> &Bn, const ChunkSrc &ncs, bool issue, const int slot) {
 #pragma unroll
         for (int i = 0; i < PER; ++i)  // slots 0..7
-            if ((i * 8) / PER == slot && issue)
-                issue_win(Bn, ncs, i);
+            if (!kCopier && (i * 8) / PER == slot && issue)
+                issue_win(Bn, ncs, NW * i, w + NW * i, woff[i]);
     };
     // copies at slots 0..7: after (a) steps 0..3 and (c) tiles 0..3
     auto phase1 = [&](ScanBuf<NW> &B, ScanBuf<NW> &Bn, const ChunkSrc &ncs, bool issue) {
@@ -550,7 +624,7 @@ __device__ __forceinline__ void scan_body(const ScanArgs &p, const ScanJob &job,
     };
 
     auto compute = [&](ScanBuf<NW> &B, int c, ScanBuf<NW> &Bn, bool more) {
-        const ChunkSrc ncs = chunk_src(more ? c + 1 : c);
+        const ChunkSrc ncs = chunk_src_v(more ? c + 1 : c, true);
         phase1(B, Bn, ncs, more);
         phase2(B, c);
     };
@@ -562,7 +636,9 @@ __device__ __forceinline__ void scan_body(const ScanArgs &p, const ScanJob &job,
     // state loads the compiler may have ordered either way are in flight: wait for all.
     const bool keep_stores = do_out;
     auto chunk_barrier = [&](bool first) {
-        if (keep_stores && !first) {
+        if constexpr (kCopier) {  // the copy wave has waited for the copies
+            lds_barrier_inflight();
+        } else if (keep_stores && !first) {
             asm volatile("" ::: "memory");
             __builtin_amdgcn_s_waitcnt(0x0074);  // vmcnt(4) lgkmcnt(0)
             __builtin_amdgcn_s_barrier();
@@ -684,7 +760,7 @@ __global__ __launch_bounds__(512) void gdn_prefill_scan8_kernel(ScanArgs p)
 }
 
 template <bool SEG>
-__global__ __launch_bounds__(256) void gdn_prefill_scan4_kernel(ScanArgs p)
+__global__ __launch_bounds__(320) void gdn_prefill_scan4_kernel(ScanArgs p)
 {
     __shared__ ScanBuf<4> bufA, bufB;
     scan_kernel_body<4, SEG>(p, bufA, bufB);
