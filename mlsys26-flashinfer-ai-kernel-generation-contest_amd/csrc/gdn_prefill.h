@@ -421,6 +421,10 @@ struct PrepArgs {
     const int32_t *header, *chunk_tok0, *chunk_len;
     char *records;
     int HQK, HV, ratio;
+    // q/k head slots per (chunk, v-head group): HQK, or 8 where HQK divides 8 and a single
+    // sequence is scanned whole (head g on XCD g, the other slots' workgroups leave at once;
+    // the grid then has a workgroup for every unit)
+    int gpad;
     float scale;
     // Self-planned launch (1 <= N <= kSelfPlanMax; no plan kernel): every workgroup finds
     // its units' chunks from cu_seqlens itself, the last block writes the tables the scan reads

@@ -149,8 +149,8 @@ __device__ __forceinline__ void prep_body(const PrepArgs &p, PrepSmem<VH> &sm)
         self_plan(p, sm, wv, l);
     // (values read from LDS are uniform here; readfirstlane tells the compiler so, or every
     // branch on them would become a divergent one)
-    const int nunits =
-        (p.self_plan ? __builtin_amdgcn_readfirstlane(sm.s_total) : p.header[0]) * p.HQK * ngrp;
+    const int nch = p.self_plan ? __builtin_amdgcn_readfirstlane(sm.s_total) : p.header[0];
+    const int nunits = nch * p.gpad * ngrp;
     // Waves are dealt to the 4 SIMDs round-robin: the second v-head takes the blocks in
     // reverse, so each SIMD pairs a heavy column block (w = 0) with a light one.
     const int hv = wv >> 2, w = hv & 1 ? 3 - (wv & 3) : (wv & 3);
@@ -161,10 +161,12 @@ __device__ __forceinline__ void prep_body(const PrepArgs &p, PrepSmem<VH> &sm)
     };
     auto unit = [&](int u) {
         Unit r;
-        const int grp = u / ngrp, hg = u % ngrp;
-        r.c = grp / p.HQK;
-        r.g = grp % p.HQK;
-        r.h = r.g * p.ratio + hg * VH + hv;
+        // q/k heads fastest: workgroups go to the 8 XCDs round-robin, so a head's units are on
+        // the XCD of its scan workgroups (whose L2 then holds their records, K and Q)
+        const int grp = u / p.gpad;
+        r.c = grp % nch;
+        r.g = u % p.gpad;
+        r.h = r.g * p.ratio + grp / nch * VH + hv;
         if (p.self_plan) {
             // the owner of chunk c is the last sequence whose first chunk is <= c (first
             // chunks never decrease; an empty sequence shares its successor's first chunk)
@@ -475,7 +477,7 @@ __device__ __forceinline__ void prep_body(const PrepArgs &p, PrepSmem<VH> &sm)
     };
 
     int u = blockIdx.x;
-    if (u >= nunits)
+    if (u >= nunits || u % p.gpad >= p.HQK)
         return;
     Unit U = unit(u);
     uint32_t a_in = 0, b_in = 0;
