@@ -4,8 +4,11 @@
 // marshalling cost about 30 us per call, ten times a small decode kernel; this path
 // costs about 1 us.
 //
+// decode_alloc() / prefill_alloc() take the calls that leave output or new_state to the callee:
+// they allocate what is missing as the Python path does and go on to decode() / prefill().
+//
 // decode() / prefill() return 0 after a successful launch and 1 when the call needs the
-// general Python path (default outputs to allocate, empty inputs, layouts the kernels
+// general Python path (empty inputs, layouts the kernels
 // cannot read or write in place, in-place with a token axis or other strides, a stream
 // being captured into a graph (prefill: that path gives each graph its own workspace),
 // or anything else they do not accept): that path then validates again and raises the
@@ -16,6 +19,7 @@
 // entry points come from libgdn_hip.so as function pointers handed over by init().
 #include <torch/extension.h>
 
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
 #include <cstring>
@@ -279,6 +283,74 @@ int64_t prefill(const at::Tensor &q, const at::Tensor &k, const at::Tensor &v,
     return 0;
 }
 
+using MaybeTensor = c10::optional<at::Tensor>;
+using MaybePair = c10::optional<std::tuple<at::Tensor, at::Tensor>>;
+
+// An allocation that fails leaves the tensor undefined: the call then declines, and the Python
+// path raises torch's own error.
+at::Tensor given_or_empty(const MaybeTensor &t, at::IntArrayRef sizes, at::ScalarType st,
+                          const c10::Device &dev)
+{
+    if (t.has_value() && t->defined())
+        return *t;
+    try {
+        return at::empty(sizes, at::TensorOptions().dtype(st).device(dev));
+    } catch (const c10::Error &) {
+        return at::Tensor();
+    }
+}
+
+// Calls without output or new_state. The sizes checked here are those of the allocations;
+// decode() / prefill() check the rest. nullopt: the general Python path's call.
+MaybePair decode_alloc(const at::Tensor &q, const at::Tensor &k, const at::Tensor &v,
+                       const MaybeTensor &state, const at::Tensor &A_log, const at::Tensor &a,
+                       const at::Tensor &dt_bias, const at::Tensor &b, double scale,
+                       const MaybeTensor &output, const MaybeTensor &new_state, int64_t variant)
+{
+    if (!g_decode || !q.defined() || !q.is_cuda())
+        return c10::nullopt;
+    const c10::Device dev = q.device();
+    if (!is(q, at::kBFloat16, 4, dev) || !is(v, at::kBFloat16, 4, dev) || q.size(3) != 128 ||
+        q.size(0) < 1 || q.size(1) < 1 || v.size(0) != q.size(0) || v.size(1) != q.size(1) ||
+        v.size(2) < 1 || v.size(3) != 128)
+        return c10::nullopt;
+    const c10::DeviceGuard guard(dev);
+    const at::Tensor out = given_or_empty(output, v.sizes(), at::kBFloat16, dev);
+    const at::Tensor ns =
+        given_or_empty(new_state, {q.size(0), v.size(2), 128, 128}, at::kFloat, dev);
+    if (!out.defined() || !ns.defined() ||
+        decode(q, k, v, state, A_log, a, dt_bias, b, scale, out, ns, variant) != 0)
+        return c10::nullopt;
+    return std::make_tuple(out, ns);
+}
+
+MaybePair prefill_alloc(const at::Tensor &q, const at::Tensor &k, const at::Tensor &v,
+                        const MaybeTensor &state, const at::Tensor &A_log, const at::Tensor &a,
+                        const at::Tensor &dt_bias, const at::Tensor &b,
+                        const at::Tensor &cu_seqlens, double scale, const MaybeTensor &output,
+                        const MaybeTensor &new_state, int64_t variant)
+{
+    if (!g_prefill || !q.defined() || !q.is_cuda())
+        return c10::nullopt;
+    const c10::Device dev = q.device();
+    if (!is(q, at::kBFloat16, 3, dev) || !is(v, at::kBFloat16, 3, dev) || q.size(2) != 128 ||
+        q.size(0) < 1 || v.size(0) != q.size(0) || v.size(1) < 1 || v.size(2) != 128 ||
+        !cu_seqlens.defined() || cu_seqlens.dim() != 1 || cu_seqlens.size(0) < 2)
+        return c10::nullopt;
+    const c10::DeviceGuard guard(dev);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c10::hip::getCurrentHIPStream(dev.index()).stream(), &cap) !=
+            hipSuccess || cap != hipStreamCaptureStatusNone)
+        return c10::nullopt;  // before anything is allocated for the graph
+    const at::Tensor out = given_or_empty(output, v.sizes(), at::kBFloat16, dev);
+    const at::Tensor ns = given_or_empty(
+        new_state, {cu_seqlens.size(0) - 1, v.size(1), 128, 128}, at::kFloat, dev);
+    if (!out.defined() || !ns.defined() ||
+        prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, out, ns, variant) != 0)
+        return c10::nullopt;
+    return std::make_tuple(out, ns);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
@@ -286,5 +358,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("init", &init, "hand over the C-ABI entry points (addresses from libgdn_hip.so)");
     m.def("decode", &decode, "validate a DPS gdn_decode call and launch it; 1 = not eligible");
     m.def("prefill", &prefill, "validate a DPS gdn_prefill call and launch it; 1 = not eligible");
+    m.def("decode_alloc", &decode_alloc,
+          "decode() with missing outputs allocated; (output, new_state), or None = not eligible");
+    m.def("prefill_alloc", &prefill_alloc,
+          "prefill() with missing outputs allocated; (output, new_state), or None = not eligible");
     m.def("release_workspace", &release_workspace, "drop the cached eager prefill workspaces");
 }

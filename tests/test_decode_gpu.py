@@ -329,6 +329,37 @@ def test_decode_fast_path_taken_and_exact(dev):
     assert torch.equal(out, o2) and torch.equal(ns, n2)
 
 
+@pytest.mark.parametrize("given", ["none", "output", "new_state"])
+def test_decode_fast_path_allocates_missing_outputs(dev, given):
+    """A call that leaves output or new_state (or both) to the callee: the fast path allocates
+    what is missing, returns what was given, and equals the destination-passing call."""
+    from gdn_hip import _lib
+
+    fast = _lib.fast()
+    g = decode_inputs(3, hqk=4, hv=8, seed=61).to(dev)
+    eo, en = torch.empty_like(g.v), torch.empty_like(g.state)
+    assert fast.decode(*g.args(), eo, en, 0) == 0
+    out = torch.empty_like(g.v) if given == "output" else None
+    ns = torch.empty_like(g.state) if given == "new_state" else None
+    r = fast.decode_alloc(*g.args(), out, ns, 0)
+    assert r is not None
+    o2, n2 = gdn_decode(*g.args(), output=out, new_state=ns)
+    torch.cuda.synchronize()
+    for o, n in (r, (o2, n2)):
+        assert torch.equal(o, eo) and torch.equal(n, en)
+        assert o.is_contiguous() and n.is_contiguous()
+        assert out is None or o.data_ptr() == out.data_ptr()
+        assert ns is None or n.data_ptr() == ns.data_ptr()
+    bad = list(g.args())
+    bad[2] = bad[2][:, :, :7]  # 7 v-heads over 4 q/k heads
+    assert fast.decode_alloc(*bad, None, None, 0) is None
+    with pytest.raises(ValueError, match="multiple"):
+        gdn_decode(*bad)
+    bad[0] = "q"
+    with pytest.raises(TypeError, match="q must be"):
+        gdn_decode(*bad)
+
+
 def test_decode_fast_path_declines_what_it_cannot_use(dev):
     """Calls the fast path cannot serve in place return 1 (the general path then handles
     them): a non-unit inner stride, a CPU tensor, a wrong dtype, mismatched shapes and an

@@ -674,6 +674,26 @@ def test_prefill_fast_path_taken_and_exact(dev):
     assert torch.equal(out, o3) and torch.equal(ns, n3)
 
 
+def test_prefill_fast_path_allocates_missing_outputs(dev):
+    """A prefill without output and new_state: allocated by the fast path, equal to the
+    destination-passing call; empty inputs still go to the general path."""
+    fast = _lib.fast()
+    g = prefill_inputs([70, 130], hqk=4, hv=8, seed=90, with_state=True).to(dev)
+    eo = torch.empty((200, 8, 128), dtype=torch.bfloat16, device=dev)
+    en = torch.empty_like(g.state)
+    assert fast.prefill(*g.args(), eo, en, 0) == 0
+    r = fast.prefill_alloc(*g.args(), None, None, 0)
+    assert r is not None
+    o2, n2 = gdn_prefill(*g.args(), output=eo.clone())
+    torch.cuda.synchronize()
+    for o, n in (r, (o2, n2)):
+        assert torch.equal(o, eo) and torch.equal(n, en)
+    e = prefill_inputs([0, 0], seed=2, with_state=True).to(dev)
+    assert fast.prefill_alloc(*e.args(), None, None, 0) is None
+    o, n = gdn_prefill(*e.args())
+    assert o.shape[0] == 0 and torch.equal(n, e.state)
+
+
 def test_prefill_fast_path_declines_capture_and_odd_layouts(dev):
     """Graph capture, a strided output and empty inputs go to the general path."""
     from gdn_hip import _lib
