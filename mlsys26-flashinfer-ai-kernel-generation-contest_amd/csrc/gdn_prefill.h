@@ -29,8 +29,8 @@
 //         32 state rows per wave and two workgroups per CU (gdn_prefill_wide.hip).
 //
 // Files: gdn_prefill.h (records, layouts, argument structs, shared helpers),
-// gdn_prefill_plan.hip, gdn_prefill_prep.hip, gdn_prefill_scan.hip, gdn_prefill_wide.hip (the
-// kernels) and gdn_prefill.hip (workspace layout and launches behind gdn_prefill_launch).
+// gdn_prefill_plan.hip, gdn_prefill_prep.hip, gdn_prefill_scan.hip, gdn_prefill_split.h (a
+// scan body), gdn_prefill_wide.hip (the kernels) and gdn_prefill.hip (workspace layout and launches behind gdn_prefill_launch).
 #pragma once
 
 #include "gdn_common.h"

@@ -353,7 +353,13 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
         auto scan = [&](int64_t units, bool nw4, bool wide = false) {
             const int64_t ngroups = units * HQK;
             sa.ngroups = (int)ngroups;
-            const int tph = nw4 ? 2 : 1;
+            // (sequence or job, q/k head) groups go to the XCDs in turn; workgroups per v-head:
+            // one, or two for the 4-wave scan, or four where that still fits one per CU (its
+            // kernel then takes the column-split bodies; with a smaller grid it does so when
+            // the device's job count leaves room)
+            int tph = nw4 ? 2 : 1;
+            if (nw4 && 8 * ((int64_t)4 * ratio) * ((ngroups + 7) / 8) <= num_cus(st))
+                tph = 4;
             const int64_t blocks = 8 * ((int64_t)tph * ratio) * ((ngroups + 7) / 8);
             if (ngroups > 0x7fffffff || blocks > 0x7fffffff)
                 return gdn_set_error(GDN_EINVAL, "gdn_prefill: grid too large");

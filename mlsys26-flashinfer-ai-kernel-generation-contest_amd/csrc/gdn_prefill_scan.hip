@@ -1,6 +1,7 @@
 // Prefill scan kernels: the sequential chunk recurrence, state in registers, for whole
 // sequences or segment jobs.
 #include "gdn_prefill.h"
+#include "gdn_prefill_split.h"
 
 #include <cstddef>
 
@@ -759,11 +760,42 @@ __global__ __launch_bounds__(512) void gdn_prefill_scan8_kernel(ScanArgs p)
     scan_kernel_body<8, SEG>(p, bufA, bufB);
 }
 
+// LDS of the 4-wave scan kernels: the 64-row bodies' two chunk buffers or the column-split
+// bodies' buffers.
+union Scan4Lds {
+    struct {
+        ScanBuf<4> a, b;
+    } s4;
+    SplitLds sp;
+};
+
+// The grid holds at most one workgroup per CU. When four workgroups per (job, v-head) fit it,
+// the column-split bodies take the jobs (32 state rows each), else the 64-row bodies (two).
 template <bool SEG>
 __global__ __launch_bounds__(320) void gdn_prefill_scan4_kernel(ScanArgs p)
 {
-    __shared__ ScanBuf<4> bufA, bufB;
-    scan_kernel_body<4, SEG>(p, bufA, bufB);
+    __shared__ Scan4Lds lds;
+    const int avail = (int)(gridDim.x / (32u * p.ratio)) * 8;  // q/k head groups of four per v-head
+    const int groups = SEG ? p.header[p.njob_idx] * p.HQK : p.ngroups;
+    if (groups > avail) {
+        scan_kernel_body<4, SEG>(p, lds.s4.a, lds.s4.b);
+        return;
+    }
+    ScanJob job;
+    if (!scan_job<2, SEG>(p, job))
+        return;
+    if constexpr (SEG) {
+        if (job.kind == kJobFirst && job.q < 0 && job.cb == 0)
+            split_body<false, 1, 1>(fresh_kernel_args(), job, lds.sp);
+        else if (job.kind == kJobFirst || job.kind == kJobResume)
+            split_body<true, 0, 1>(fresh_kernel_args(), job, lds.sp);
+        else if (job.kind == kJobZero)
+            split_body<true, 0, 0>(fresh_kernel_args(), job, lds.sp);
+        else
+            split_body<true, 0, 2>(fresh_kernel_args(), job, lds.sp);
+    } else {
+        split_body<false, 0, 1>(fresh_kernel_args(), job, lds.sp);
+    }
 }
 
 template __global__ void gdn_prefill_scan8_kernel<false>(ScanArgs p);

@@ -213,16 +213,17 @@ def gdn_decode(q, k, v, state, A_log, a, dt_bias, b, scale, output=None, new_sta
     """
     if scale is None or type(scale) is float:
         fast = _lib.fast()
-        if fast is not None:
-            sc = 0.0 if scale is None else scale
-            if output is None or new_state is None:
-                r = _alloc_call(fast.decode_alloc, q, k, v, state, A_log, a, dt_bias, b, sc,
-                                output, new_state, 0)
-                if r is not None:
-                    return r
-            elif fast.decode(q, k, v, state, A_log, a, dt_bias, b, sc, output, new_state,
-                             0) == 0:
+        if fast is None:
+            pass
+        elif output is not None and new_state is not None:
+            if fast.decode(q, k, v, state, A_log, a, dt_bias, b, 0.0 if scale is None else scale,
+                           output, new_state, 0) == 0:
                 return output, new_state
+        else:
+            r = _alloc_call(fast.decode_alloc, q, k, v, state, A_log, a, dt_bias, b,
+                            0.0 if scale is None else scale, output, new_state, 0)
+            if r is not None:
+                return r
     with torch.no_grad():
         P, output, new_state, copy_back, _keep = _decode_marshal(
             q, k, v, state, A_log, a, dt_bias, b, scale, output, new_state)
@@ -448,16 +449,18 @@ def gdn_prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output=
     """
     if scale is None or type(scale) is float:
         fast = _lib.fast()
-        if fast is not None:
-            sc = 0.0 if scale is None else scale
-            if output is None or new_state is None:
-                r = _alloc_call(fast.prefill_alloc, q, k, v, state, A_log, a, dt_bias, b,
-                                cu_seqlens, sc, output, new_state, _prefill_variant)
-                if r is not None:
-                    return r
-            elif fast.prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, sc, output,
-                              new_state, _prefill_variant) == 0:
+        if fast is None:
+            pass
+        elif output is not None and new_state is not None:
+            if fast.prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens,
+                            0.0 if scale is None else scale, output, new_state,
+                            _prefill_variant) == 0:
                 return output, new_state
+        else:
+            r = _alloc_call(fast.prefill_alloc, q, k, v, state, A_log, a, dt_bias, b, cu_seqlens,
+                            0.0 if scale is None else scale, output, new_state, _prefill_variant)
+            if r is not None:
+                return r
     with torch.no_grad():
         m = _prefill_marshal(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output,
                              new_state)

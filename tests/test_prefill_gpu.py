@@ -298,6 +298,23 @@ def test_prefill_many_sequences(dev, nseq):
 
 
 @pytest.mark.parametrize("lens,hqk,hv,state,gates", [
+    # four workgroups per v-head on the column-split bodies: up to one per CU (64 pairs at
+    # 256 CUs), and just above; whole sequences, segments with 0 to 3 chain steps, empty and
+    # 1-token sequences, chunk edges, an odd head ratio
+    ([1, 64, 65, 0, 127, 128, 129, 200], 4, 8, True, "mild"),
+    ([1, 64, 65, 0, 127, 128, 129, 200, 31], 4, 8, True, "mild"),
+    ([300, 65], 16, 32, False, "none"),
+    ([900, 1], 4, 8, True, "none"),
+    ([1500], 4, 8, True, "mild"),
+    ([1600], 1, 3, True, "mild"),
+    ([63], 16, 32, True, "strong"),
+])
+def test_prefill_column_split_scan(dev, lens, hqk, hv, state, gates):
+    _run(dev, prefill_inputs(lens, hqk=hqk, hv=hv, seed=sum(lens) % 89, with_state=state,
+                             gates=gates), f"column split {lens[:3]} x {hv}")
+
+
+@pytest.mark.parametrize("lens,hqk,hv,state,gates", [
     # the scan with two workgroups per CU (768 (sequence, v-head) pairs and more): chunk edges
     # and remainders, empty sequences, odd and even chunk counts, the smallest batch it takes
     ([1, 63, 64, 65, 0, 127, 128, 129, 191, 192, 193, 257, 31, 2, 320, 16, 17, 96, 64, 33, 5, 48,
