@@ -15,27 +15,57 @@ int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
 int64_t max_chunks(int64_t T, int64_t N) { return (T + kChunkH - 1) / kChunkH + N; }
 
-// Segments per sequence (the default variant only): when (sequence, v-head) pairs are too
-// few to fill 256 CUs, the largest G <= gdn::kSegMaxG whose pass-A jobs N HV (2 G - 3)
-// still fit one workgroup per CU; 1 means no segments (G = 2 would scan its halves one
-// after the other). The planner picks each sequence's count up to G from its length.
+// A scan chunk's time in k cycles (MI355X, one job per workgroup) with this many (job, v-head)
+// pairs: the column-split bodies up to 64, the 4-wave scan up to 128, the 8-wave scan. A state
+// map's chunk (no outputs) takes kSegFirstWeight of it.
+double chunk_cost(int64_t pairs) { return pairs <= 64 ? 3.6 : pairs <= 128 ? 4.4 : 6.5; }
+
+// Segments per sequence at most (the default variant only; 1: none). Segments scan a sequence's
+// parts side by side at the price of a second pass (its launch, state and first chunk: ~14 k
+// cycles) and of state maps on more CUs, whose scan may be a slower one. The largest count is
+// bounded by pass A's jobs, N HV (2 G - 3), at one workgroup per CU; G = 2 would scan its halves
+// one after the other.
+//
+// One sequence of c chunks: the G with the smallest modelled time, both passes taking the
+// planner's base(G) = (c + h (G - 1) (G - 2)) / (w + G - 1) chunks, against c chunks whole.
+// Whole prefills at 32 v-heads, cut into as many segments as pass A holds -> this rule (whole):
+// 1 x 800 34.1 -> 32.7 us, 1 x 1200 48.4 -> 43.6.
+//
+// More sequences, whose lengths only the device knows (its planner picks each one's count up to
+// this G): the largest G where they are long, on average or together. Else none are cut, since a
+// pass A without jobs still costs 1.7 us and a cut made for a slower scan more (8 sequences of 64
+// to 1024 at 8 v-heads 38.8 -> 37.1 us, 4 such 30.4 -> 28.9, 2 of 700 to 1000 39.2 -> 36.2, 2 of
+// 800 to 900 at 32 48.6 -> 38.8). Where pass A needs the 8-wave scan the whole scan is 1.5 to
+// 1.8 times as fast per chunk, so only very long sequences are cut.
 int seg_count(int64_t T, int64_t N, int64_t HV)
 {
     // (the job planner runs one sequence per lane in the self-planned prep kernel)
     if (T <= 0 || N <= 0 || N > gdn::kSelfPlanMax || N * HV * 3 > 256)
         return 1;
-    int64_t G = 3;
-    while (G < gdn::kSegMaxG && N * HV * (2 * (G + 1) - 3) <= 256)
-        ++G;
-    // No sequence has more than ceil(T / 64) chunks, and the planner cuts one of c chunks
-    // into at most min(G, c / kSegMinChunks, G*(c)) segments, G* its closed-form optimum
-    // (rising with c; +1 for the device's float rounding). Capacities sized for that count
-    // are tight for a single sequence (1 x 1024 at 8 v-heads: 4 segments instead of 16),
-    // and below 3 no sequence is cut at all: one whole-sequence scan.
-    const int64_t cmax = (T + kChunkH - 1) / kChunkH;
+    const int64_t cmax = (T + kChunkH - 1) / kChunkH;  // no sequence has more chunks
     const double w = gdn::kSegFirstWeight, h = 0.5 * gdn::kSegChainChunks;
-    const int64_t gs = (int64_t)(1.0 - w + std::sqrt(w * w + w + (double)cmax / h)) + 1;
-    G = std::min({G, cmax / gdn::kSegMinChunks, gs});
+    int64_t G = 1;
+    double best = cmax * chunk_cost(HV);
+    for (int64_t g = 3; g <= gdn::kSegMaxG && N * HV * (2 * g - 3) <= 256 && g <= cmax / gdn::kSegMinChunks; ++g) {
+        if (N > 1) {
+            G = g;
+            continue;
+        }
+        const double base = (cmax + h * (g - 1) * (g - 2)) / (w + g - 1);
+        const double cost = base * (w * chunk_cost(HV * (2 * g - 3)) + chunk_cost(HV * (g - 1))) + 14.0;
+        if (cost < best) {
+            best = cost;
+            G = g;
+        }
+    }
+    if (N > 1) {
+        if (N * HV * 3 > 128 ? T < 2560 * N : T < 1024 * N && T < 2560)
+            return 1;
+        // the planner cuts c chunks into at most G*(c) segments, its closed-form optimum (rising
+        // with c; +1 for the device's float rounding): capacities sized for that are tight
+        const int64_t gs = (int64_t)(1.0 - w + std::sqrt(w * w + w + (double)cmax / h)) + 1;
+        G = std::min(G, gs);
+    }
     return G >= 3 ? (int)G : 1;
 }
 
