@@ -16,9 +16,10 @@ int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 int64_t max_chunks(int64_t T, int64_t N) { return (T + kChunkH - 1) / kChunkH + N; }
 
 // A scan chunk's time in k cycles (MI355X, one job per workgroup) with this many (job, v-head)
-// pairs: the column-split bodies up to 64, the 4-wave scan up to 128, the 8-wave scan. A state
-// map's chunk (no outputs) takes kSegFirstWeight of it.
-double chunk_cost(int64_t pairs) { return pairs <= 64 ? 3.6 : pairs <= 128 ? 4.4 : 6.5; }
+// pairs: the column-split bodies up to 64, the 4-wave scan up to 128, the 8-wave scan (6.5 on
+// its own; 7.6 fits the best of the counts measured below). A state map's chunk (no outputs)
+// takes kSegFirstWeight of it.
+double chunk_cost(int64_t pairs) { return pairs <= 64 ? 3.6 : pairs <= 128 ? 4.4 : 7.6; }
 
 // Segments per sequence at most (the default variant only; 1: none). Segments scan a sequence's
 // parts side by side at the price of a second pass (its launch, state and first chunk: ~14 k
@@ -28,8 +29,10 @@ double chunk_cost(int64_t pairs) { return pairs <= 64 ? 3.6 : pairs <= 128 ? 4.4
 //
 // One sequence of c chunks: the G with the smallest modelled time, both passes taking the
 // planner's base(G) = (c + h (G - 1) (G - 2)) / (w + G - 1) chunks, against c chunks whole.
-// Whole prefills at 32 v-heads, cut into as many segments as pass A holds -> this rule (whole):
-// 1 x 800 34.1 -> 32.7 us, 1 x 1200 48.4 -> 43.6.
+// Whole prefills, as many segments as pass A holds -> this rule: at 8 v-heads 1 x 4096 64.1 ->
+// 51.1 us (9 segments; 5 59.4), 1 x 8192 90.5 -> 74.8 (9), 1 x 16384 131.3 -> 128.5 (9; 12 136.0);
+// at 32 v-heads 1 x 800 33.9 -> 32.5 (whole), 1 x 1200 47.7 -> 42.1 (3), 1 x 1600 52.4 -> 48.8
+// (3), 1 x 4096 93 (5; 3 97).
 //
 // More sequences, whose lengths only the device knows (its planner picks each one's count up to
 // this G): the largest G where they are long, on average or together. Else none are cut, since a

@@ -113,16 +113,23 @@ __device__ __forceinline__ void self_plan(const PrepArgs &p, PrepSmem<VH> &sm, i
         if (q.seg_G >= 3)  // every lane of the wave takes part
             plan_jobs(q, order, sm.s_first, sm.s_t0, sm.s_len, l);
         if (q.whole_cus > 0) {
-            // Whole sequences, both scans launched. The 4-wave scan spreads each (sequence,
-            // v-head) over two CUs: a chunk takes ~0.74 of the 8-wave scan's time, but
-            // costs 1.5 times the CU time. It is the faster while its average load per CU
-            // (chunk-times over all jobs) stays below the longest sequence, which bounds
-            // both scans from below (measured on MI355X at load / longest: 0.71 -13 %,
-            // 1.02 -4 %, 1.06 +3 %, 1.27 +6 %); 0.9 leaves the close calls to the 8-wave
-            // scan.
+            // Whole sequences, both scans launched. The 8-wave scan has a CU for each (sequence,
+            // v-head) and takes the longest sequence's chunks; a chunk of the 4-wave scan is
+            // 1.5 times as fast, but its twice as many workgroups share the CUs: besides the
+            // longest sequence, the mean load per CU and the two jobs that meet on the CU filled
+            // last (longest first) bound it. Measured on MI355X at 8 v-heads, 8-wave -> 4-wave,
+            // with bound / longest: 20 of 64 to 1024 65.4 -> 49.4 us (0.69), 24 of 1 to 200 27.8
+            // -> 27.0 (1.1), 30 of 100 to 700 62.1 -> 57.5 (1.2), 24 of 500 to 700 61.8 -> 65.4
+            // (1.8), 17 of 400 40.3 -> 45.8 (2).
             const float cmax = wave_max_nonneg((float)nck);
             const float load4 = 2.f * (float)sm.s_total * (float)q.HO / (float)q.whole_cus;
-            const bool use4 = load4 <= 0.9f * cmax;
+            auto of_rank = [&](int r) {  // chunks of the sequence of rank r
+                const uint64_t m = __ballot(l < q.N && rank == r);
+                const int c = __builtin_amdgcn_readlane(nck, m ? __builtin_ctzll(m) : 0);
+                return m ? c : 0;
+            };
+            const int meet = of_rank((q.whole_cus - 1) / (2 * q.HO)) + of_rank(q.whole_cus / (2 * q.HO));
+            const bool use4 = fmaxf(load4, (float)meet) <= 1.25f * cmax;
             if (l == 0) {
                 q.header[4] = use4 ? q.N : 0;
                 q.header[5] = use4 ? 0 : q.N;
