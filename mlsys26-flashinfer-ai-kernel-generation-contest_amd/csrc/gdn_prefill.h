@@ -15,7 +15,7 @@
 // Launches on the caller's stream:
 //   plan  (1 + Z workgroups): sequence -> chunk tables from cu_seqlens on the device
 //         (no host sync), longest-first sequence order, and zero-fill of output rows
-//         that belong to no sequence. Skipped for 1 to 64 sequences, where the prep
+//         that belong to no sequence. Skipped for 1 to 126 sequences, where the prep
 //         kernel does the same work itself (PrepArgs::self_plan).
 //   prep  (chunks x q/k heads): K K^T and Q K^T on MFMA, gates, cumulative log
 //         decay, T = (I + A)^-1 (16x16 diagonal blocks by fp32 substitution,
@@ -173,6 +173,21 @@ __device__ __forceinline__ float quad_bcast(float x)
 __device__ __forceinline__ int64_t load_cu(const void *cu, int cu64, int i)
 {
     return cu64 ? ((const int64_t *)cu)[i] : (int64_t)((const int32_t *)cu)[i];
+}
+
+// cu[i] and cu[i + 1], both loads in flight at once
+__device__ __forceinline__ void load_cu2(const void *cu, int cu64, int i, int64_t &a, int64_t &b)
+{
+    if (cu64) {
+        const int64_t *p = (const int64_t *)cu + i;
+        a = p[0];
+        b = p[1];
+    } else {
+        const int32_t *p = (const int32_t *)cu + i;
+        const int32_t x = p[0], y = p[1];
+        a = x;
+        b = y;
+    }
 }
 
 // Segment jobs. When (sequence, v-head) pairs are too few to fill the GPU, a long sequence
@@ -434,7 +449,10 @@ struct PrepArgs {
     PlanArgs plan;
 };
 
-constexpr int kSelfPlanMax = 64;  // one sequence per lane of a wave
+// Two sequences per lane of a wave, less two: the table then just fits the 80 KB of LDS that
+// two prep workgroups per CU leave each.
+constexpr int kSelfPlanMax = 126;
+constexpr int kSegSeqMax = 64;  // segments: the job planner takes one sequence per lane
 
 // ------------------------------------------------------------------------- scan
 struct ScanArgs {

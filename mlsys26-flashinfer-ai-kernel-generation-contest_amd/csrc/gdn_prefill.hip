@@ -43,7 +43,7 @@ double chunk_cost(int64_t pairs) { return pairs <= 64 ? 3.6 : pairs <= 128 ? 4.4
 int seg_count(int64_t T, int64_t N, int64_t HV)
 {
     // (the job planner runs one sequence per lane in the self-planned prep kernel)
-    if (T <= 0 || N <= 0 || N > gdn::kSelfPlanMax || N * HV * 3 > 256)
+    if (T <= 0 || N <= 0 || N > gdn::kSegSeqMax || N * HV * 3 > 256)
         return 1;
     const int64_t cmax = (T + kChunkH - 1) / kChunkH;  // no sequence has more chunks
     const double w = gdn::kSegFirstWeight, h = 0.5 * gdn::kSegChainChunks;
@@ -260,8 +260,9 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
     const bool c4_only = L.capC * HV <= 128;
     pa.seg_c4 = G > 1 && !c4_only ? (int)(128 / HV) : 0;
     pa.jobs = G > 1 ? (int32_t *)(ws + L.jobs) : nullptr;
-    // Up to 64 sequences the prep kernel plans for itself (one dependent launch fewer:
-    // the plan kernel's ~5 us sat on the critical path, mostly cu_seqlens load latency).
+    // Up to 126 sequences the prep kernel plans for itself (one dependent launch fewer: the
+    // plan kernel's 5 to 6 us sat on the critical path, mostly cu_seqlens load latency; 100
+    // sequences of 1 to 130 at 32 v-heads 179.1 -> 176.8 us, 100 of 64 to 160 at 8 78.2 -> 74.2).
     const bool prep_runs = L.nc > 0 && T > 0;
     const bool self_plan = prep_runs && N >= 1 && N <= gdn::kSelfPlanMax;
     // Whole sequences, 129 to 256 (sequence, v-head) pairs: either scan can be the faster,
@@ -269,7 +270,7 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
     // and the self-planning prep kernel gives the sequences to one of them; the other
     // launch finds none (~1.5-2 us for its up to 512 workgroups, one per CU at a time for
     // their LDS). Above 256 pairs the 8-wave scan alone (the 4-wave one rarely wins there).
-    const bool whole_dual = G == 1 && p->variant == 0 && self_plan && (int64_t)N * HV > 128 &&
+    const bool whole_dual = G == 1 && p->variant == 0 && self_plan && N <= gdn::kSegSeqMax && (int64_t)N * HV > 128 &&
                             (int64_t)N * HV <= 256;
     // With three (sequence, v-head) pairs per CU and more, of at most six chunks on average, a
     // pair's start and end (state and first chunk in, state out) weigh as much as its chunks:

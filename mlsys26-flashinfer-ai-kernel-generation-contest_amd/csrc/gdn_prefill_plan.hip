@@ -1,4 +1,4 @@
-// Prefill plan kernel (more than 64 sequences): sequence -> chunk tables from cu_seqlens on
+// Prefill plan kernel (more than 126 sequences): sequence -> chunk tables from cu_seqlens on
 // the device, longest-first sequence order, zero-fill of rows outside every sequence.
 #include "gdn_prefill.h"
 
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void gdn_prefill_plan_kernel(PlanArgs p)
             }
         }
         // (segment job tables come from the prep kernel: segments are used up to 64
-        // sequences only, where the prep kernel plans for itself)
+        // sequences only, where it plans for itself)
         return;
     }
     // Zero-fill output rows of tokens outside [cu[0], cu[N]).

@@ -38,10 +38,9 @@ struct PrepSmem {
     u32x4 XA[VH][4][64];  // X_w in A-operand layout, by lane, split4
     u32x4 AO[VH][6][64];  // off-diagonal A_im (m < i) as XA; index i(i-1)/2 + m
     float Ms[4 * VH][16][16];  // per wave: -A_ww rows, X_w, then T' staging
-    // self-planned launches: sequence n's first chunk (clamped to nc; nc past the N
-    // sequences), first token and length; the chunk total and the covered tokens [g0, g1)
-    int32_t s_first[kSelfPlanMax], s_t0[kSelfPlanMax], s_len[kSelfPlanMax];
-    int32_t s_total, s_g0, s_g1, s_pad;
+    // self-planned launches: sequence n's first chunk (clamped to nc; nc past the N sequences),
+    // its first token (entry N: the last one's end) and the chunk total
+    int32_t s_first[kSelfPlanMax + 1], s_t0[kSelfPlanMax + 1], s_total;
 };
 
 constexpr int kGateWave = 3;  // column block with no work after the barrier
@@ -55,54 +54,71 @@ template <int VH>
 __device__ __forceinline__ void self_plan(const PrepArgs &p, PrepSmem<VH> &sm, int wv, int l)
 {
     const PlanArgs &q = p.plan;
+    // Lane l plans sequence l and, above 64 sequences, 64 + l. A sequence's end is the next
+    // one's first token, not before its own.
+    auto len_of = [&](int n) { return max(sm.s_t0[n + 1] - sm.s_t0[n], 0); };
+    const bool two = q.N > 64;
     if (wv == 0) {
-        int t0 = 0, ln = 0;
-        int64_t nck = 0, braw = 0;
-        if (l < q.N) {
-            int64_t a = load_cu(q.cu, q.cu64, l), b = load_cu(q.cu, q.cu64, l + 1);
-            braw = b;
-            a = a < 0 ? 0 : (a > q.T ? q.T : a);
-            b = b < a ? a : (b > q.T ? q.T : b);
-            t0 = (int)a;
-            ln = (int)(b - a);
-            nck = (ln + kC - 1) / kC;
-        }
-        const int64_t incl = wave_prefix_sum_i64(nck), first = incl - nck;
-        sm.s_first[l] = l < q.N ? (int32_t)(first < q.nc ? first : q.nc) : q.nc;
-        sm.s_t0[l] = t0;
-        sm.s_len[l] = ln;
-        if (l == 63)
-            sm.s_total = (int32_t)(incl < q.nc ? incl : q.nc);
-        // Cross-lane reads stay in wave-uniform control flow: inside a lane-conditional
-        // branch the compiler may reuse the source register in lanes outside the branch.
-        const int last = q.N - 1;
-        const int64_t b_hi = __builtin_amdgcn_readlane((int)(braw >> 32), last),
-                      b_lo = (uint32_t)__builtin_amdgcn_readlane((int)braw, last);
-        const int64_t g1 = (b_hi << 32) | b_lo;
-        const int g0 = __builtin_amdgcn_readlane(t0, 0);  // cu[0] clamped to [0, T]
-        if (l == 0) {
-            sm.s_g0 = g0;
-            sm.s_g1 = (int32_t)(g1 < g0 ? g0 : (g1 > q.T ? q.T : g1));
-        }
+        auto clamp_tok = [&](int64_t x) { return (int)(x < 0 ? 0 : (x > q.T ? q.T : x)); };
+        auto set = [&](int n, int64_t before) {  // returns the chunks up to the set's last lane
+            int64_t nck = 0;
+            if (n < q.N) {
+                int64_t a, b;
+                load_cu2(q.cu, q.cu64, n, a, b);
+                const int ca = clamp_tok(a), cb = clamp_tok(b);
+                sm.s_t0[n] = ca;
+                if (n == q.N - 1)
+                    sm.s_t0[q.N] = cb;
+                nck = (max(cb - ca, 0) + kC - 1) / kC;
+            }
+            const int64_t incl = before + wave_prefix_sum_i64(nck), first = incl - nck;
+            if (n <= kSelfPlanMax)
+                sm.s_first[n] = n < q.N ? (int32_t)(first < q.nc ? first : q.nc) : q.nc;
+            // Cross-lane reads stay in wave-uniform control flow: inside a lane-conditional
+            // branch the compiler may reuse the source register in lanes outside the branch.
+            return ((int64_t)__builtin_amdgcn_readlane((int)(incl >> 32), 63) << 32) |
+                   (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        };
+        int64_t total = set(l, 0);
+        if (two)
+            total = set(64 + l, total);
+        if (l == 0)
+            sm.s_total = (int32_t)(total < q.nc ? total : q.nc);
     }
     __syncthreads();
     if (blockIdx.x == gridDim.x - 1 && wv == 0) {
-        const int first = sm.s_first[l], t0 = sm.s_t0[l], ln = sm.s_len[l];
-        const int nck = (ln + kC - 1) / kC;
-        int rank = 0;
-        for (int m = 0; m < q.N; ++m) {
+        // (lanes past the N sequences: no chunks)
+        auto chunks = [&](int n) { return n < q.N ? (len_of(n) + kC - 1) / kC : 0; };
+        const int nck = chunks(l), nck1 = two ? chunks(64 + l) : 0;
+        int rank = 0, rank1 = 0;
+        for (int m = 0; m < min(q.N, 64); ++m) {
             const int o = __builtin_amdgcn_readlane(nck, m);
             rank += (o > nck) || (o == nck && m < l);
+            rank1 += o >= nck1;
+        }
+        for (int m = 64; m < q.N; ++m) {
+            const int o = __builtin_amdgcn_readlane(nck1, m - 64);
+            rank += o > nck;
+            rank1 += (o > nck1) || (o == nck1 && m < 64 + l);
         }
         // the second K buffer is not written before the first unit's barrier
-        int32_t *order = (int32_t *)sm.K[1];
+        int32_t *order = (int32_t *)sm.K[1], *lens = order + 64;
+        auto put = [&](int n, int r) {
+            const int t0 = sm.s_t0[n], ln = len_of(n), first = sm.s_first[n];
+            q.seq_tok0[n] = t0;
+            q.seq_len[n] = ln;
+            q.seq_chunk0[n] = first;
+            *(int4 *)(q.seq_rank + 4 * r) = int4{n, t0, ln, first};
+        };
         if (l < q.N) {
-            q.seq_tok0[l] = t0;
-            q.seq_len[l] = ln;
-            q.seq_chunk0[l] = first;
-            *(int4 *)(q.seq_rank + 4 * rank) = int4{l, t0, ln, first};
-            order[rank] = l;
+            put(l, rank);
+            if (!two) {
+                order[rank] = l;
+                lens[l] = len_of(l);
+            }
         }
+        if (64 + l < q.N)
+            put(64 + l, rank1);
         if (l == 0) {
             q.seq_chunk0[q.N] = sm.s_total;
             q.header[0] = sm.s_total;
@@ -111,7 +127,7 @@ __device__ __forceinline__ void self_plan(const PrepArgs &p, PrepSmem<VH> &sm, i
             q.header[2] = q.N;
         }
         if (q.seg_G >= 3)  // every lane of the wave takes part
-            plan_jobs(q, order, sm.s_first, sm.s_t0, sm.s_len, l);
+            plan_jobs(q, order, sm.s_first, sm.s_t0, lens, l);
         if (q.whole_cus > 0) {
             // Whole sequences, both scans launched. The 8-wave scan has a CU for each (sequence,
             // v-head) and takes the longest sequence's chunks; a chunk of the 4-wave scan is
@@ -136,7 +152,7 @@ __device__ __forceinline__ void self_plan(const PrepArgs &p, PrepSmem<VH> &sm, i
             }
         }
     }
-    const int g0 = sm.s_g0, g1 = sm.s_g1, gap = g0 + (q.T - g1);
+    const int g0 = sm.s_t0[0], g1 = max(g0, sm.s_t0[q.N]), gap = g0 + (q.T - g1);
     if (gap > 0) {
         const int per_tok = q.HO * (kDK / 8);
         const u32x4 z = {0u, 0u, 0u, 0u};
@@ -180,11 +196,18 @@ __device__ __forceinline__ void prep_body(const PrepArgs &p, PrepSmem<VH> &sm)
         if (p.self_plan) {
             // the owner of chunk c is the last sequence whose first chunk is <= c (first
             // chunks never decrease; an empty sequence shares its successor's first chunk)
-            const int f = sm.s_first[l];
-            const int n = __popcll(__ballot(f <= r.c)) - 1;
-            const int i = r.c - __builtin_amdgcn_readlane(f, n);
-            r.tok0 = __builtin_amdgcn_readfirstlane(sm.s_t0[n]) + kC * i;
-            r.len = min(kC, __builtin_amdgcn_readfirstlane(sm.s_len[n]) - kC * i);
+            int ll = l;
+            asm volatile("" : "+v"(ll));  // (no table address kept in a register across units)
+            const int f = sm.s_first[ll];
+            int n = __popcll(__ballot(f <= r.c)) - 1, fc;
+            if (p.plan.N > 64) {
+                n += __popcll(__ballot(sm.s_first[min(64 + ll, kSelfPlanMax)] <= r.c));
+                fc = __builtin_amdgcn_readfirstlane(sm.s_first[n]);
+            } else {
+                fc = __builtin_amdgcn_readlane(f, n);
+            }
+            r.tok0 = __builtin_amdgcn_readfirstlane(sm.s_t0[n]) + kC * (r.c - fc);
+            r.len = min(kC, __builtin_amdgcn_readfirstlane(sm.s_t0[n + 1]) - r.tok0);
         } else {
             r.tok0 = p.chunk_tok0[r.c];
             r.len = p.chunk_len[r.c];

@@ -328,6 +328,19 @@ def test_prefill_wide_scan(dev, lens, hqk, hv, state, gates):
                              gates=gates), f"wide scan {len(lens)} x {hv}")
 
 
+@pytest.mark.parametrize("nseq", [63, 64, 65, 125, 126, 127])
+def test_prefill_planning_limits(dev, nseq):
+    """One and two planned sequences per lane, and the plan kernel above 126: empty and short
+    sequences, chunk edges, tokens before the first and after the last, both cu_seqlens types;
+    every path gives the same chunk numbering, so equal inputs give equal bits."""
+    lens = [(0, 1, 64, 65, 130, 20)[i % 6] for i in range(nseq)]
+    inp = prefill_inputs(lens, hqk=2, hv=4, seed=nseq, with_state=True, gates="mild",
+                         cu_dtype=torch.int64 if nseq % 2 else torch.int32, pad_tokens=7)
+    inp.cu_seqlens += 3  # three tokens before the first sequence
+    inp.cu_seqlens[-1] -= 3 if lens[-1] >= 3 else 0
+    _run(dev, inp, f"planning limit N={nseq}")
+
+
 @pytest.mark.parametrize("nseq", [3, 64, 300])
 def test_prefill_gap_before_first_sequence(dev, nseq):
     """cu_seqlens[0] > 0: the leading tokens belong to no sequence and read as zero."""
