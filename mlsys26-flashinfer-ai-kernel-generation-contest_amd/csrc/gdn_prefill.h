@@ -30,7 +30,8 @@
 //
 // Files: gdn_prefill.h (records, layouts, argument structs, shared helpers),
 // gdn_prefill_plan.hip, gdn_prefill_prep.hip, gdn_prefill_scan.hip, gdn_prefill_split.h (a
-// scan body), gdn_prefill_wide.hip (the kernels) and gdn_prefill.hip (workspace layout and launches behind gdn_prefill_launch).
+// scan body), gdn_prefill_wide.hip (the kernels) and gdn_prefill.hip (workspace layout and
+// launches behind gdn_prefill_launch).
 #pragma once
 
 #include "gdn_common.h"

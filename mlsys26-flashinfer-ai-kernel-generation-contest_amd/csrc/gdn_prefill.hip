@@ -269,7 +269,8 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
     // depending on the longest sequence, which only the device knows. Both are launched
     // and the self-planning prep kernel gives the sequences to one of them; the other
     // launch finds none (~1.5-2 us for its up to 512 workgroups, one per CU at a time for
-    // their LDS). Above 256 pairs the 8-wave scan alone (the 4-wave one rarely wins there).
+    // their LDS). Above 256 pairs the 8-wave scan alone (the 4-wave one rarely
+    // wins there), or the wide one below.
     const bool whole_dual = G == 1 && p->variant == 0 && self_plan && N <= gdn::kSegSeqMax && (int64_t)N * HV > 128 &&
                             (int64_t)N * HV <= 256;
     // With three (sequence, v-head) pairs per CU and more, of at most six chunks on average, a
