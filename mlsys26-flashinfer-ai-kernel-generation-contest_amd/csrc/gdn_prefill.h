@@ -249,10 +249,36 @@ struct PlanArgs {
     // CUs): the planner gives the sequences to the 4-wave launch (header[4] = N, header[5] = 0)
     // when it is the faster, else to the 8-wave launch (header[4] = 0, header[5] = N)
     int whole_cus;
+    // wide_cus > 0 (many short sequences: the wide scan and the queued 8-wave scan both
+    // launched, this many CUs): the planner gives the sequences to the wide one (header[6] = N,
+    // header[5] = 0) or, where the longest one alone would take too long there, to the other
+    // (header[5] = N, header[6] = 0), whose job queues (header[8 .. 15]) it empties
+    int wide_cus;
     int32_t *jobs;
 };
 
 constexpr int kPlanSortMax = 512;
+constexpr int kQueueIdx = 8;  // header[8 .. 15]: next job slot per XCD of the queued 8-wave scan
+
+// The choice between the wide scan and the 8-wave scan, from the longest sequence's chunks and
+// the total. Chunks go through the chip 2 to 13 % faster in the wide scan, but a sequence's own
+// go 1.29 times slower (3.4 against 2.65 us each, the longest's chain alone), so it wins while
+// the longest sequence stays below 0.65 of the load per CU, a (sequence, v-head)'s start and
+// end counted as two chunks. Measured on MI355X over 107 batches of 26 to 500 sequences at 4 to
+// 32 v-heads, 1 to 4 of them long: wide / 8-wave 0.87 to 0.98 up to a ratio of 0.55, 1.04 to
+// 1.13 at 0.9 to 1, 1.2 to 1.3 above 1.3; this line never costs more than 1.1 %. Whole prefills
+// without the choice -> with it: 5000 and 40 of 64 tokens at 32 v-heads 315 -> 253 us, 16384 and
+// 99 of 64 at 8 874 -> 682, 1024 and 30 of 64 at 32 87 -> 74; the launch that finds nothing costs
+// 1.8 us (100 of 64 at 32 155 -> 157).
+__device__ inline void choose_wide(const PlanArgs &p, float cmax, float total)
+{
+    const float load = (total + 2.f * (float)p.N) * (float)p.HO / (float)p.wide_cus;
+    const bool wide = cmax <= 0.65f * load;
+    p.header[5] = wide ? 0 : p.N;
+    p.header[6] = wide ? p.N : 0;
+    for (int x = 0; x < 8; ++x)
+        p.header[kQueueIdx + x] = 0;
+}
 
 // Maximum over the 64 lanes of non-negative values (the prefix pattern of
 // wave_prefix_sum_i64; lane 63 holds the total), returned to every lane.
@@ -474,6 +500,7 @@ struct ScanArgs {
     // lo units (seg_mt, kMtUnits).
     const int32_t *jobs;
     int job_first, njob_idx;
+    int32_t *queue;  // the queued 8-wave scan's next slot per XCD
     float *seg_sin, *seg_r, *seg_mt;
 };
 
@@ -484,14 +511,14 @@ struct ScanJob {
     int grp, wi, n, tok0, len, c0, kind, cb, ce, q, steps, last;
 };
 
-// Finds this workgroup's job (SEG: in the segment job table); false when it has none.
+// Finds the job of workgroup pid (SEG: in the segment job table); false when it has none.
 template <int NW, bool SEG>
-__device__ __forceinline__ bool scan_job(const ScanArgs &p, ScanJob &j)
+__device__ __forceinline__ bool scan_job(const ScanArgs &p, ScanJob &j, int pid)
 {
     constexpr int TPH = 8 / NW;  // workgroups per (sequence, v-head)
     // Workgroups of one (sequence, q/k head) share K, Q through L2: one XCD for them all
     // (workgroup ids are dealt to the 8 XCDs round-robin).
-    const int pid = blockIdx.x, xcd = pid & 7, slot = pid >> 3;
+    const int xcd = pid & 7, slot = pid >> 3;
     const int gsz = TPH * p.ratio;
     j.wi = slot % gsz;
     j.grp = (slot / gsz) * 8 + xcd;
@@ -623,6 +650,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void
 gdn_prefill_prep2_kernel(PrepArgs p);
 template <bool SEG>
 __global__ __launch_bounds__(512) void gdn_prefill_scan8_kernel(ScanArgs p);
+__global__ __launch_bounds__(512) void gdn_prefill_scan8q_kernel(ScanArgs p);
 template <bool SEG>
 __global__ __launch_bounds__(320) void gdn_prefill_scan4_kernel(ScanArgs p);
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void

@@ -280,10 +280,13 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
     // 181 us, 64 of 128 162 -> 145, 40 of 64 to 200 108 -> 100, 24 of 1 to 100 56 -> 51, 100 of
     // 64 to 256 at 8 v-heads 97 -> 91. Fewer pairs gain nothing (20 of 300 to 500 at 32 v-heads
     // 114.5 -> 115.5, 16 of 64 to 1024 124 -> 128: two long jobs share a CU's time), nor do
-    // longer sequences (32 of 512 209 -> 212, 64 of 1000 728 -> 743).
+    // longer sequences (32 of 512 209 -> 212, 64 of 1000 728 -> 743). A long sequence among the
+    // short ones, which only the device knows of, makes the planner take the 8-wave scan after
+    // all (choose_wide).
     const bool wide = G == 1 && p->variant == 0 && (int64_t)N * HV >= 3 * (int64_t)num_cus(st) &&
                       T <= 384 * (int64_t)N;
     pa.whole_cus = whole_dual ? num_cus(st) : 0;
+    pa.wide_cus = wide ? num_cus(st) : 0;
     gdn_begin_launches();
     int rc = 0;
     if (!self_plan) {
@@ -379,6 +382,7 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
         sa.jobs = nullptr;
         sa.job_first = 0;
         sa.njob_idx = 0;
+        sa.queue = pa.header + gdn::kQueueIdx;
         sa.seg_sin = G > 1 ? (float *)(ws + L.seg_sin) : nullptr;
         sa.seg_r = G > 1 ? (float *)(ws + L.seg_r) : nullptr;
         sa.seg_mt = G > 1 ? (float *)(ws + L.seg_mt) : nullptr;
@@ -436,8 +440,18 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
                 sa.njob_idx = 5;
                 rc = scan(N, false);
             }
+        } else if (wide) {
+            sa.njob_idx = 6;
+            rc = scan(N, false, true);
+            if (rc == 0) {
+                sa.njob_idx = 5;
+                const int64_t cus = num_cus(st);  // one workgroup per CU, at least one per queue
+                hipLaunchKernelGGL(gdn::gdn_prefill_scan8q_kernel,
+                                   dim3((unsigned)(8 * std::max<int64_t>(cus / 8, 1))), dim3(512), 0, st, sa);
+                rc = gdn_check_launch("gdn_prefill_scan8q_kernel");
+            }
         } else {
-            rc = scan(N, nw4, wide);
+            rc = scan(N, nw4);
         }
         if (rc)
             return rc;

@@ -17,10 +17,12 @@ __global__ __launch_bounds__(256) void gdn_prefill_plan_kernel(PlanArgs p)
         __shared__ int32_t s_first[kPlanSortMax], s_end[kPlanSortMax], s_t0[kPlanSortMax],
             s_len[kPlanSortMax];
         __shared__ int64_t s_carry;
+        __shared__ float s_cmax[4];  // each wave's longest sequence, in chunks
         const bool par = p.N <= kPlanSortMax;
         if (tid == 0)
             s_carry = 0;
         __syncthreads();
+        float cmax = 0.f;
         for (int base = 0; base < p.N; base += 256) {
             const int n = base + tid;
             int nck = 0, t0 = 0, ln = 0;
@@ -31,6 +33,7 @@ __global__ __launch_bounds__(256) void gdn_prefill_plan_kernel(PlanArgs p)
                 t0 = (int)a;
                 ln = (int)(b - a);
                 nck = (ln + kC - 1) / kC;
+                cmax = fmaxf(cmax, (float)nck);
                 p.seq_tok0[n] = t0;
                 p.seq_len[n] = ln;
                 if (n < kPlanSortMax)
@@ -71,6 +74,15 @@ __global__ __launch_bounds__(256) void gdn_prefill_plan_kernel(PlanArgs p)
             const int32_t total = (int32_t)(s_carry < p.nc ? s_carry : p.nc);
             p.seq_chunk0[p.N] = total;
             p.header[0] = total;
+        }
+        if (p.wide_cus > 0) {
+            const float m = wave_max_nonneg(cmax);
+            if ((tid & 63) == 0)
+                s_cmax[tid >> 6] = m;
+            __syncthreads();
+            if (tid == 0)
+                choose_wide(p, fmaxf(fmaxf(s_cmax[0], s_cmax[1]), fmaxf(s_cmax[2], s_cmax[3])),
+                            (float)s_carry);
         }
         if (par) {  // chunk c belongs to the first sequence whose chunks end after c
             __syncthreads();

@@ -151,6 +151,11 @@ __device__ __forceinline__ void self_plan(const PrepArgs &p, PrepSmem<VH> &sm, i
                 q.header[5] = use4 ? 0 : q.N;
             }
         }
+        if (q.wide_cus > 0) {
+            const float cmax = wave_max_nonneg((float)max(nck, nck1));
+            if (l == 0)
+                choose_wide(q, cmax, (float)sm.s_total);
+        }
     }
     const int g0 = sm.s_t0[0], g1 = max(g0, sm.s_t0[q.N]), gap = g0 + (q.T - g1);
     if (gap > 0) {

@@ -37,9 +37,13 @@ namespace gdn {
 // INST tags an instance: the whole-sequence body inside a segment kernel is instance 1, so
 // each instance is used by one kernel only (hipcc's host pass rejects a second kernel's use
 // of an instance of this device-only template: "substitution failure").
-template <int NW, bool SEG, int INST = 0, int OUTS = -1>
+// on_last: called by every wave as it starts the job's last chunk (not for a job without one).
+struct NoHook {
+    __device__ __forceinline__ void operator()() const {}
+};
+template <int NW, bool SEG, int INST = 0, int OUTS = -1, class F = NoHook>
 __device__ __forceinline__ void scan_body(const ScanArgs &p, const ScanJob &job, ScanBuf<NW> &BA,
-                                          ScanBuf<NW> &BB)
+                                          ScanBuf<NW> &BB, F on_last = F{})
 {
     constexpr int TPH = 8 / NW;  // workgroups per (sequence, v-head)
     const int grp = job.grp, wi = job.wi, n = job.n, tok0 = job.tok0, len = job.len,
@@ -650,10 +654,14 @@ __device__ __forceinline__ void scan_body(const ScanArgs &p, const ScanJob &job,
     };
     for (int c = cb; c < ce; c += 2) {
         chunk_barrier(c == cb);  // chunk c is in BA; every wave is done with BB
+        if (c + 1 >= ce)
+            on_last();
         compute(BA, c, BB, c + 1 < ce);
         if (c + 1 >= ce)
             break;
         chunk_barrier(false);
+        if (c + 2 >= ce)
+            on_last();
         compute(BB, c + 1, BA, c + 2 < ce);
     }
 
@@ -736,7 +744,7 @@ __device__ __forceinline__ void scan_kernel_body(const ScanArgs &p, ScanBuf<NW> 
                                                  ScanBuf<NW> &BB)
 {
     ScanJob job;
-    if (!scan_job<NW, SEG>(p, job))
+    if (!scan_job<NW, SEG>(p, job, blockIdx.x))
         return;
     if constexpr (SEG) {
         if (job.kind == kJobFirst && job.q < 0 && job.cb == 0) {
@@ -758,6 +766,36 @@ __global__ __launch_bounds__(512) void gdn_prefill_scan8_kernel(ScanArgs p)
 {
     __shared__ ScanBuf<8> bufA, bufB;
     scan_kernel_body<8, SEG>(p, bufA, bufB);
+}
+
+// The 8-wave whole-sequence scan behind the wide one (choose_wide, gdn_prefill.h): one workgroup
+// per CU (a multiple of eight), which starts on the job of its own index and then takes jobs
+// from its XCD's queue until that is empty: longest first to whichever workgroup is free, as the
+// hardware hands them out in a grid of one workgroup per job. Such a grid, of several workgroups
+// per CU, costs 3 to 6 us where the planner gave every sequence to the wide scan; this one 1.8.
+__global__ __launch_bounds__(512) void gdn_prefill_scan8q_kernel(ScanArgs p)
+{
+    __shared__ ScanBuf<8> bufA, bufB;
+    __shared__ int32_t s_slot;
+    const int xcd = blockIdx.x & 7;
+    int slot = blockIdx.x >> 3;
+    auto pull = [&] { return (int)(gridDim.x >> 3) + atomicAdd(p.queue + xcd, 1); };
+    for (;;) {
+        ScanJob job;
+        // (a slot past the last job ends the workgroup: its queue is handed out)
+        if (slot > (0x7fffffff >> 3) || !scan_job<8, false>(p, job, 8 * slot + xcd))
+            return;
+        int next = -1;  // thread 0: the next slot, pulled during the job's last chunk
+        scan_body<8, false, 2>(fresh_kernel_args(), job, bufA, bufB, [&] {
+            if (threadIdx.x == 0)
+                next = pull();
+        });
+        if (threadIdx.x == 0)
+            s_slot = next >= 0 ? next : pull();  // (an empty sequence has no chunk)
+        __syncthreads();  // every wave is done with the buffers
+        slot = __builtin_amdgcn_readfirstlane(s_slot);
+        __syncthreads();  // s_slot is free again
+    }
 }
 
 // LDS of the 4-wave scan kernels: the 64-row bodies' two chunk buffers or the column-split
@@ -782,7 +820,7 @@ __global__ __launch_bounds__(320) void gdn_prefill_scan4_kernel(ScanArgs p)
         return;
     }
     ScanJob job;
-    if (!scan_job<2, SEG>(p, job))
+    if (!scan_job<2, SEG>(p, job, blockIdx.x))
         return;
     if constexpr (SEG) {
         if (job.kind == kJobFirst && job.q < 0 && job.cb == 0)

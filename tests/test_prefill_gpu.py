@@ -328,6 +328,45 @@ def test_prefill_wide_scan(dev, lens, hqk, hv, state, gates):
                              gates=gates), f"wide scan {len(lens)} x {hv}")
 
 
+def _run_with_header(dev, inp, label, ints=16):
+    """One prefill through the C entry point against the oracle; returns the first ints of
+    the workspace header, where the planner leaves its job counts."""
+    from gdn_hip.api import _prefill_marshal
+    ref_out, ref_ns = _oracle(inp)
+    g = inp.to(dev)
+    hv = g.v.shape[1]
+    out = torch.empty(g.v.shape, dtype=torch.bfloat16, device=dev)
+    ns = torch.empty((len(inp.seqlens), hv, 128, 128), dtype=torch.float32, device=dev)
+    P, _, _, copy_back, keep, stream = _prefill_marshal(*g.args(), out, ns)
+    assert not copy_back
+    print(f"[{label}] launching", flush=True)
+    rc = _lib.load().gdn_prefill_launch(ctypes.byref(P), ctypes.c_void_p(stream.cuda_stream))
+    assert rc == 0, _lib.load().gdn_last_error()
+    torch.cuda.synchronize()
+    header = keep[-1][:4 * ints].view(torch.int32).cpu().tolist()
+    print(f"[{label}] header {header}", flush=True)
+    _check(out, ns, ref_out, ref_ns, label)
+    return header
+
+
+@pytest.mark.parametrize("lens,hqk,hv,wide", [
+    ([64] * 96, 4, 8, True),
+    ([1500] + [40] * 95, 4, 8, False),              # a long prompt among short ones
+    ([900, 0, 700] + [33] * 127, 2, 6, False),      # the same through the plan kernel
+    ([20] * 519 + [600], 1, 2, False),              # too many to sort: the long one comes last
+    ([20] * 520, 1, 2, True),
+])
+def test_prefill_wide_scan_choice(dev, lens, hqk, hv, wide):
+    """768 (sequence, v-head) pairs and more, short on average: the planner gives the sequences
+    to the wide scan (header[6]) unless the longest one's chain alone would take longer there
+    than the whole batch in the 8-wave scan (header[5]), whose job queues then hand out every
+    job once."""
+    inp = prefill_inputs(lens, hqk=hqk, hv=hv, seed=len(lens), with_state=True, gates="mild")
+    header = _run_with_header(dev, inp, f"wide choice N={len(lens)}")
+    n = len(lens)
+    assert (header[5], header[6]) == ((0, n) if wide else (n, 0))
+
+
 @pytest.mark.parametrize("nseq", [63, 64, 65, 125, 126, 127])
 def test_prefill_planning_limits(dev, nseq):
     """One and two planned sequences per lane, and the plan kernel above 126: empty and short
