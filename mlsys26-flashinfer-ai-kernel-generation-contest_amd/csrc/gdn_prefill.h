@@ -245,9 +245,9 @@ struct PlanArgs {
     // counts them in header[2] for the 4-wave launch, a larger one in header[3] for the
     // 8-wave launch, and the other launch finds no job.
     int seg_G, seg_capA, seg_c4;
-    // whole_cus > 0 (whole sequences, the 4-wave and the 8-wave scan both launched, this many
-    // CUs): the planner gives the sequences to the 4-wave launch (header[4] = N, header[5] = 0)
-    // when it is the faster, else to the 8-wave launch (header[4] = 0, header[5] = N)
+    // whole_cus > 0 (whole sequences, either width of the scan, this many CUs): the planner
+    // gives the sequences to the 4-wave form (header[4] = N, header[5] = 0) when it is the
+    // faster, else to the 8-wave form (header[4] = 0, header[5] = N)
     int whole_cus;
     // wide_cus > 0 (many short sequences: the wide scan and the queued 8-wave scan both
     // launched, this many CUs): the planner gives the sequences to the wide one (header[6] = N,
@@ -651,6 +651,7 @@ gdn_prefill_prep2_kernel(PrepArgs p);
 template <bool SEG>
 __global__ __launch_bounds__(512) void gdn_prefill_scan8_kernel(ScanArgs p);
 __global__ __launch_bounds__(512) void gdn_prefill_scan8q_kernel(ScanArgs p);
+__global__ __launch_bounds__(512) void gdn_prefill_scan_any_kernel(ScanArgs p);
 template <bool SEG>
 __global__ __launch_bounds__(320) void gdn_prefill_scan4_kernel(ScanArgs p);
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void

@@ -265,12 +265,10 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
     // sequences of 1 to 130 at 32 v-heads 179.1 -> 176.8 us, 100 of 64 to 160 at 8 78.2 -> 74.2).
     const bool prep_runs = L.nc > 0 && T > 0;
     const bool self_plan = prep_runs && N >= 1 && N <= gdn::kSelfPlanMax;
-    // Whole sequences, 129 to 256 (sequence, v-head) pairs: either scan can be the faster,
-    // depending on the longest sequence, which only the device knows. Both are launched
-    // and the self-planning prep kernel gives the sequences to one of them; the other
-    // launch finds none (~1.5-2 us for its up to 512 workgroups, one per CU at a time for
-    // their LDS). Above 256 pairs the 8-wave scan alone (the 4-wave one rarely
-    // wins there), or the wide one below.
+    // Whole sequences, 129 to 256 (sequence, v-head) pairs: either width of the scan can be the
+    // faster, depending on the longest sequence, which only the device knows: the self-planning
+    // prep kernel chooses. Above 256 pairs the 8-wave scan alone (the 4-wave one rarely wins
+    // there), or the wide one below.
     const bool whole_dual = G == 1 && p->variant == 0 && self_plan && N <= gdn::kSegSeqMax && (int64_t)N * HV > 128 &&
                             (int64_t)N * HV <= 256;
     // With three (sequence, v-head) pairs per CU and more, of at most six chunks on average, a
@@ -434,12 +432,10 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
                 rc = scan(L.capC, false);
             }
         } else if (whole_dual) {
-            sa.njob_idx = 4;
-            rc = scan(N, true);
-            if (rc == 0) {
-                sa.njob_idx = 5;
-                rc = scan(N, false);
-            }
+            sa.ngroups = N * HQK;  // at most 256 (sequence, v-head) pairs
+            const unsigned blocks = 8 * 2 * ratio * ((sa.ngroups + 7) / 8);
+            hipLaunchKernelGGL(gdn::gdn_prefill_scan_any_kernel, dim3(blocks), dim3(512), 0, st, sa);
+            rc = gdn_check_launch("gdn_prefill_scan_any_kernel");
         } else if (wide) {
             sa.njob_idx = 6;
             rc = scan(N, false, true);

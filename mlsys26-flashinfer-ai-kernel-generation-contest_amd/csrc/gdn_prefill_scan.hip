@@ -836,6 +836,27 @@ __global__ __launch_bounds__(320) void gdn_prefill_scan4_kernel(ScanArgs p)
     }
 }
 
+// Whole sequences at the planner's choice of width, in one launch: 4 waves and the copy wave (the
+// other three leave at once), two workgroups per (sequence, v-head), for header[4] sequences, or
+// 8 waves and one workgroup for header[5] of them; one of the two counts is zero. A launch for
+// each width left one of them without a job: 6 sequences of 80 to 180 tokens at 32 v-heads 27.0
+// -> 25.3 us, 20 of 400 at 8 43.2 -> 41.6, 32 of 64 to 1024 at 8 78.0 -> 76.4.
+__global__ __launch_bounds__(512) void gdn_prefill_scan_any_kernel(ScanArgs p)
+{
+    __shared__ ScanBuf<8> bufA, bufB;
+    ScanJob job;
+    const int n4 = p.header[4], n8 = p.header[5];
+    if (n4 > 0) {
+        // (a scalar branch: the three waves end here, and barriers count those that are left)
+        if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) > 4)
+            return;
+        if (scan_job<4, false>(p, job, blockIdx.x))
+            scan_body<4, false, 3>(fresh_kernel_args(), job, (ScanBuf<4> &)bufA, (ScanBuf<4> &)bufB);
+    } else if (n8 > 0 && scan_job<8, false>(p, job, blockIdx.x)) {
+        scan_body<8, false, 3>(fresh_kernel_args(), job, bufA, bufB);
+    }
+}
+
 template __global__ void gdn_prefill_scan8_kernel<false>(ScanArgs p);
 template __global__ void gdn_prefill_scan8_kernel<true>(ScanArgs p);
 template __global__ void gdn_prefill_scan4_kernel<false>(ScanArgs p);
