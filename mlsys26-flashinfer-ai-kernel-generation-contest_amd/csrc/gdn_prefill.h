@@ -228,6 +228,20 @@ constexpr int kSegMaxG = 16;                // segments per sequence at most
 constexpr float kSegFirstWeight = 0.83f;
 constexpr float kSegChainChunks = 0.9f;
 
+// Up to this many (job, v-head) pairs a scan runs 4 waves per workgroup, two workgroups a pair
+constexpr int kPairs4 = 128;
+
+// A scan chunk's time in k cycles (MI355X, one job per workgroup) with this many (job, v-head)
+// pairs: the column-split bodies up to 64, the 4-wave scan up to 128, the 8-wave scan (6.5 on
+// its own; 7.6 fits the best of the segment counts measured in gdn_prefill.hip). A state map's
+// chunk (no outputs) takes kSegFirstWeight of it.
+__host__ __device__ inline float chunk_cost(int64_t pairs)
+{
+    return pairs <= 64 ? 3.6f : pairs <= kPairs4 ? 4.4f : 7.6f;
+}
+constexpr float kSegPassCost = 14.f;  // a second pass: its launch, state and first chunk
+constexpr float kSegEmptyPass = 4.f;  // a pass without a job (1.7 us)
+
 // ------------------------------------------------------------------------- plan
 struct PlanArgs {
     const void *cu;
@@ -240,11 +254,8 @@ struct PlanArgs {
     int64_t o_st, o_sh;
     // segments (seg_G >= 3): at most seg_G segments per sequence; job entries of kJobInts
     // ints, pass A from jobs[0], pass C from jobs[kJobInts seg_capA]; counts in header[1]
-    // (pass A) and header[2] (pass C). seg_c4 > 0: pass C is launched twice, with 4 and with
-    // 8 waves per workgroup; a plan with at most seg_c4 pass-C jobs (128 (job, v-head) pairs)
-    // counts them in header[2] for the 4-wave launch, a larger one in header[3] for the
-    // 8-wave launch, and the other launch finds no job.
-    int seg_G, seg_capA, seg_c4;
+    // (pass A) and header[2] (pass C)
+    int seg_G, seg_capA;
     // whole_cus > 0 (whole sequences, either width of the scan, this many CUs): the planner
     // gives the sequences to the 4-wave form (header[4] = N, header[5] = 0) when it is the
     // faster, else to the 8-wave form (header[4] = 0, header[5] = N)
@@ -305,9 +316,10 @@ __device__ __forceinline__ float wave_max_nonneg(float x)
 // seg_G and len / kSegMinChunks, below the minimum of 2 base(G) over real G,
 // G* = 1 - w + sqrt(w^2 + w + len / h) with w = kSegFirstWeight, h = kSegChainChunks / 2.
 // Shorter sequences stay whole and run in whichever pass they lengthen least; a whole
-// job is a kJobFirst entry without a slot, which either pass runs. When the longest
-// sequence scanned whole is no longer than the two spans plus one chunk time (a second
-// pass's start), nothing is cut and every sequence runs whole in pass C.
+// job is a kJobFirst entry without a slot, which either pass runs. When the longest sequence
+// scanned whole takes no longer than the two spans and the second pass's start, each at the
+// chunk time of the scan that its number of jobs calls for, nothing is cut and every sequence
+// runs whole in pass C. (One sequence: the host has weighed that.)
 // Pass A lists every segment 0 and whole sequence first (rank order), then the state maps;
 // slots q .. q + G - 2 of a cut sequence hold S_in(1) and M_s, R_s of the middle segments
 // s (slot q + s - 1).
@@ -384,7 +396,15 @@ __device__ inline void plan_jobs(const PlanArgs &p, const int32_t *order, const 
             in_c |= uint64_t(1) << i;
         }
     }
-    const bool whole_all = cmax <= spanA + spanC + 1.f;
+    // (pass A of this plan: a segment 0 or a whole job of every sequence but those in pass C,
+    // and two maps for each middle segment)
+    const int extra = act && G > 1 ? G - 2 : 0;
+    const int64_t mid = wave_prefix_sum_i64(extra), ncut = wave_prefix_sum_i64(act && G > 1);
+    const int nmid = (int)__builtin_amdgcn_readlane((int)mid, 63),
+              nc = (int)__builtin_amdgcn_readlane((int)ncut, 63), inC = __popcll(in_c);
+    const float cut = w * chunk_cost((int64_t)(p.N - inC + 2 * nmid) * p.HO) * spanA +
+                      chunk_cost((int64_t)(nc + nmid + inC) * p.HO) * spanC + kSegPassCost - kSegEmptyPass;
+    const bool whole_all = nc == 0 || (p.N > 1 && chunk_cost((int64_t)p.N * p.HO) * cmax <= cut);
     const bool whole = whole_all || G == 1;
     const bool wc = whole_all || ((in_c >> lane) & 1);
     // job counts -> offsets (exclusive prefix sums in rank order)
@@ -421,10 +441,8 @@ __device__ inline void plan_jobs(const PlanArgs &p, const int32_t *order, const 
         }
     }
     if (lane == 0) {
-        const bool c8 = p.seg_c4 > 0 && totC > p.seg_c4;
         p.header[1] = totF + totM;
-        p.header[2] = c8 ? 0 : totC;
-        p.header[3] = c8 ? totC : 0;
+        p.header[2] = totC;
     }
 }
 
@@ -492,12 +510,12 @@ struct ScanArgs {
     const int32_t *header, *seq_chunk0, *seq_tok0, *seq_len, *seq_rank;
     const char *records;
     int HQK, HV, ratio, ngroups;
-    // Segment jobs (jobs != nullptr): the grid walks entries jobs[kJobInts (job_first + e)]
-    // for e < header[njob_idx] instead of whole sequences. Whole sequences (jobs == nullptr)
-    // with njob_idx > 0: only the sequences of rank < header[njob_idx] are scanned (the
-    // planner hands all or none of them to this launch). Slot buffers hold one 128 x 128
-    // fp32 matrix per (slot, v-head): S_in(1) (seg_sin), R_s (seg_r), or M_s as bf16 hi /
-    // lo units (seg_mt, kMtUnits).
+    int split_groups;  // (job, q/k head) groups whose four workgroups per v-head find a CU each
+    // Segment jobs: the grid walks entries jobs[kJobInts (job_first + e)] for e <
+    // header[njob_idx] instead of whole sequences. Slot buffers hold one 128 x 128 fp32 matrix
+    // per (slot, v-head): S_in(1) (seg_sin), R_s (seg_r), or M_s as bf16 hi / lo units (seg_mt,
+    // kMtUnits). Whole sequences in the wide scan or the queued one: those of rank <
+    // header[njob_idx] are scanned (the planner hands all or none of them to a launch).
     const int32_t *jobs;
     int job_first, njob_idx;
     int32_t *queue;  // the queued 8-wave scan's next slot per XCD
@@ -511,9 +529,12 @@ struct ScanJob {
     int grp, wi, n, tok0, len, c0, kind, cb, ce, q, steps, last;
 };
 
-// Finds the job of workgroup pid (SEG: in the segment job table); false when it has none.
+constexpr int kAllJobs = 0x7fffffff;
+
+// Finds the job of workgroup pid (SEG: in the segment job table) among the first njob; false
+// when it has none.
 template <int NW, bool SEG>
-__device__ __forceinline__ bool scan_job(const ScanArgs &p, ScanJob &j, int pid)
+__device__ __forceinline__ bool scan_job(const ScanArgs &p, ScanJob &j, int pid, int njob)
 {
     constexpr int TPH = 8 / NW;  // workgroups per (sequence, v-head)
     // Workgroups of one (sequence, q/k head) share K, Q through L2: one XCD for them all
@@ -536,7 +557,7 @@ __device__ __forceinline__ bool scan_job(const ScanArgs &p, ScanJob &j, int pid)
         const int e = j.grp / p.HQK;
         const int4 *je = (const int4 *)(p.jobs + kJobInts * (p.job_first + e));
         const int4 j0 = je[0], j1 = je[1], j2 = je[2];
-        if (e >= p.header[p.njob_idx])
+        if (e >= njob)
             return false;
         j.n = j0.x;
         j.kind = j0.y;
@@ -552,7 +573,7 @@ __device__ __forceinline__ bool scan_job(const ScanArgs &p, ScanJob &j, int pid)
         // ranks below ngroups / HQK = N all have an entry: load it with the count
         const int e = j.grp / p.HQK;
         const int4 r = *(const int4 *)(p.seq_rank + 4 * e);
-        if (p.njob_idx > 0 && e >= p.header[p.njob_idx])
+        if (e >= njob)
             return false;
         j.n = r.x;
         j.tok0 = r.y;
@@ -641,19 +662,18 @@ struct ScanBuf {
 
 // ------------------------------------------------------------------------- kernels
 // Defined in gdn_prefill_plan.hip, gdn_prefill_prep.hip, gdn_prefill_scan.hip and
-// gdn_prefill_wide.hip; the scan4 / scan8 kernels are instantiated there for SEG = false (whole sequences) and true
-// (segment jobs).
+// gdn_prefill_wide.hip; scan_any is instantiated there for SEG = false (whole sequences) and
+// true (segment jobs).
 __global__ __launch_bounds__(256) void gdn_prefill_plan_kernel(PlanArgs p);
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void
 gdn_prefill_prep1_kernel(PrepArgs p);
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void
 gdn_prefill_prep2_kernel(PrepArgs p);
-template <bool SEG>
 __global__ __launch_bounds__(512) void gdn_prefill_scan8_kernel(ScanArgs p);
 __global__ __launch_bounds__(512) void gdn_prefill_scan8q_kernel(ScanArgs p);
-__global__ __launch_bounds__(512) void gdn_prefill_scan_any_kernel(ScanArgs p);
-template <bool SEG>
 __global__ __launch_bounds__(320) void gdn_prefill_scan4_kernel(ScanArgs p);
+template <bool SEG>
+__global__ __launch_bounds__(512) void gdn_prefill_scan_any_kernel(ScanArgs p);
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 gdn_prefill_scanw_kernel(ScanArgs p);
 

@@ -15,12 +15,6 @@ int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
 int64_t max_chunks(int64_t T, int64_t N) { return (T + kChunkH - 1) / kChunkH + N; }
 
-// A scan chunk's time in k cycles (MI355X, one job per workgroup) with this many (job, v-head)
-// pairs: the column-split bodies up to 64, the 4-wave scan up to 128, the 8-wave scan (6.5 on
-// its own; 7.6 fits the best of the counts measured below). A state map's chunk (no outputs)
-// takes kSegFirstWeight of it.
-double chunk_cost(int64_t pairs) { return pairs <= 64 ? 3.6 : pairs <= 128 ? 4.4 : 7.6; }
-
 // Segments per sequence at most (the default variant only; 1: none). Segments scan a sequence's
 // parts side by side at the price of a second pass (its launch, state and first chunk: ~14 k
 // cycles) and of state maps on more CUs, whose scan may be a slower one. The largest count is
@@ -34,12 +28,19 @@ double chunk_cost(int64_t pairs) { return pairs <= 64 ? 3.6 : pairs <= 128 ? 4.4
 // at 32 v-heads 1 x 800 33.9 -> 32.5 (whole), 1 x 1200 47.7 -> 42.1 (3), 1 x 1600 52.4 -> 48.8
 // (3), 1 x 4096 93 (5; 3 97).
 //
-// More sequences, whose lengths only the device knows (its planner picks each one's count up to
-// this G): the largest G where they are long, on average or together. Else none are cut, since a
-// pass A without jobs still costs 1.7 us and a cut made for a slower scan more (8 sequences of 64
-// to 1024 at 8 v-heads 38.8 -> 37.1 us, 4 such 30.4 -> 28.9, 2 of 700 to 1000 39.2 -> 36.2, 2 of
-// 800 to 900 at 32 48.6 -> 38.8). Where pass A needs the 8-wave scan the whole scan is 1.5 to
-// 1.8 times as fast per chunk, so only very long sequences are cut.
+// More sequences: only the device knows their lengths. It weighs its plan against scanning every
+// sequence whole (plan_jobs); what is decided here is whether it may cut, since a pass A without
+// a job costs ~1.7 us. The most there is to gain is one sequence of all T tokens among empty
+// ones, the most to lose that launch in a batch of equal lengths: segments where the first, as
+// a share of its call, is at least kSegOdds times the second. Whole prefills, every sequence
+// whole below a mean length -> this rule: 1980 + 20 tokens at 8 v-heads 59.8 -> 39.5 us, 2400 + 3
+// of 20 70.2 -> 45.0, 6000 + 5 of 100 155.5 -> 90.8, 15000 + 9 of 200 380 -> 260, 3000 + 20 at
+// 32 89.9 -> 72.4, 1500 + 300 at 16 49.2 -> 37.0; with nothing to cut 6 of 1000 at 8 40.0 ->
+// 41.8, 2048 + 1100 at 32 69.1 -> 71.1, and 3 of 700 at 8, offered for what 2100 tokens in one
+// sequence would gain, 28.9 -> 30.8. (8 of 64 to 1024 at 8 are not offered: 36.4.)
+constexpr double kSegOdds = 3.75;
+constexpr double kCallRest = 45.0;  // k cycles of a call besides its chunks (prep, starts)
+
 int seg_count(int64_t T, int64_t N, int64_t HV)
 {
     // (the job planner runs one sequence per lane in the self-planned prep kernel)
@@ -47,28 +48,25 @@ int seg_count(int64_t T, int64_t N, int64_t HV)
         return 1;
     const int64_t cmax = (T + kChunkH - 1) / kChunkH;  // no sequence has more chunks
     const double w = gdn::kSegFirstWeight, h = 0.5 * gdn::kSegChainChunks;
+    const double whole = cmax * gdn::chunk_cost(N * HV);
+    // the planner cuts c chunks into at most G*(c) segments, its closed-form optimum (rising with
+    // c; +1 for the device's float rounding): capacities sized for that are tight
+    const int64_t gs = (int64_t)(1.0 - w + std::sqrt(w * w + w + (double)cmax / h)) + 1;
     int64_t G = 1;
-    double best = cmax * chunk_cost(HV);
+    double best = whole;
     for (int64_t g = 3; g <= gdn::kSegMaxG && N * HV * (2 * g - 3) <= 256 && g <= cmax / gdn::kSegMinChunks; ++g) {
-        if (N > 1) {
-            G = g;
-            continue;
-        }
+        if (N > 1 && g > gs)
+            break;
         const double base = (cmax + h * (g - 1) * (g - 2)) / (w + g - 1);
-        const double cost = base * (w * chunk_cost(HV * (2 * g - 3)) + chunk_cost(HV * (g - 1))) + 14.0;
-        if (cost < best) {
+        const double cost = base * (w * gdn::chunk_cost(HV * (2 * g - 3 + N - 1)) + gdn::chunk_cost(HV * (g - 1))) +
+                            gdn::kSegPassCost;
+        if (cost < best || N > 1) {
             best = cost;
             G = g;
         }
     }
-    if (N > 1) {
-        if (N * HV * 3 > 128 ? T < 2560 * N : T < 1024 * N && T < 2560)
-            return 1;
-        // the planner cuts c chunks into at most G*(c) segments, its closed-form optimum (rising
-        // with c; +1 for the device's float rounding): capacities sized for that are tight
-        const int64_t gs = (int64_t)(1.0 - w + std::sqrt(w * w + w + (double)cmax / h)) + 1;
-        G = std::min(G, gs);
-    }
+    if (N > 1 && (whole - best) * (whole / N + kCallRest) < kSegOdds * gdn::kSegEmptyPass * (whole + kCallRest))
+        return 1;
     return G >= 3 ? (int)G : 1;
 }
 
@@ -250,15 +248,9 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
     // Whole sequences: 4 scan waves per workgroup (two workgroups per (sequence, v-head))
     // when there are at most 128 (sequence, v-head) pairs, else 8 (129 to 256 pairs: the
     // device picks, whole_dual below). Variants: 1 forces 4 waves, 2 forces 8.
-    const bool nw4 = p->variant == 1 || (p->variant == 0 && (int64_t)N * HV <= 128);
+    const bool nw4 = p->variant == 1 || (p->variant == 0 && (int64_t)N * HV <= gdn::kPairs4);
     pa.seg_G = G;
     pa.seg_capA = (int)L.capA;
-    // Pass C: the 4-wave kernel (two workgroups per (job, v-head), spread over twice the CUs)
-    // when its job capacity fits 128 pairs; otherwise both kernels are launched and the
-    // planner gives the jobs to the 4-wave one whenever the plan's pass C fits 128 pairs
-    // (every plan that cuts nothing, for one), else to the 8-wave one.
-    const bool c4_only = L.capC * HV <= 128;
-    pa.seg_c4 = G > 1 && !c4_only ? (int)(128 / HV) : 0;
     pa.jobs = G > 1 ? (int32_t *)(ws + L.jobs) : nullptr;
     // Up to 126 sequences the prep kernel plans for itself (one dependent launch fewer: the
     // plan kernel's 5 to 6 us sat on the critical path, mostly cu_seqlens load latency; 100
@@ -269,7 +261,7 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
     // faster, depending on the longest sequence, which only the device knows: the self-planning
     // prep kernel chooses. Above 256 pairs the 8-wave scan alone (the 4-wave one rarely wins
     // there), or the wide one below.
-    const bool whole_dual = G == 1 && p->variant == 0 && self_plan && N <= gdn::kSegSeqMax && (int64_t)N * HV > 128 &&
+    const bool whole_dual = G == 1 && p->variant == 0 && self_plan && N <= gdn::kSegSeqMax && (int64_t)N * HV > gdn::kPairs4 &&
                             (int64_t)N * HV <= 256;
     // With three (sequence, v-head) pairs per CU and more, of at most six chunks on average, a
     // pair's start and end (state and first chunk in, state out) weigh as much as its chunks:
@@ -384,70 +376,56 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
         sa.seg_sin = G > 1 ? (float *)(ws + L.seg_sin) : nullptr;
         sa.seg_r = G > 1 ? (float *)(ws + L.seg_r) : nullptr;
         sa.seg_mt = G > 1 ? (float *)(ws + L.seg_mt) : nullptr;
-        // 8 waves per workgroup = one (sequence, v-head) each, two waves per SIMD; with
-        // few (sequence, v-head) pairs, 4 waves and two workgroups per pair spread the
-        // state rows over twice as many CUs. variant: 1 forces 4 waves, 2 forces 8.
-        auto scan = [&](int64_t units, bool nw4, bool wide = false) {
+        // 8 waves per workgroup = one (sequence, v-head) each, two waves per SIMD; with few
+        // (sequence, v-head) pairs, 4 waves and two workgroups per pair (or four, where that still
+        // fits one per CU: column-split bodies) spread the state rows over more CUs. (sequence or
+        // job, q/k head) groups go to the XCDs in turn.
+        const int64_t cus = num_cus(st);
+        sa.split_groups = (int)(8 * (cus / (32 * (int64_t)ratio)));
+        auto blocks_of = [&](int64_t groups, int tph) { return 8 * ((int64_t)tph * ratio) * ((groups + 7) / 8); };
+        auto launch = [&](void (*kernel)(gdn::ScanArgs), int64_t units, int64_t blocks, int threads) {
             const int64_t ngroups = units * HQK;
             sa.ngroups = (int)ngroups;
-            // (sequence or job, q/k head) groups go to the XCDs in turn; workgroups per v-head:
-            // one, or two for the 4-wave scan, or four where that still fits one per CU (its
-            // kernel then takes the column-split bodies; with a smaller grid it does so when
-            // the device's job count leaves room)
-            int tph = nw4 ? 2 : 1;
-            if (nw4 && 8 * ((int64_t)4 * ratio) * ((ngroups + 7) / 8) <= num_cus(st))
-                tph = 4;
-            const int64_t blocks = 8 * ((int64_t)tph * ratio) * ((ngroups + 7) / 8);
             if (ngroups > 0x7fffffff || blocks > 0x7fffffff)
                 return gdn_set_error(GDN_EINVAL, "gdn_prefill: grid too large");
-            // (scan4: four compute waves and the copy wave)
-            const dim3 grid((unsigned)blocks), bw(256), b4(320), b8(512);
-            if (wide)
-                hipLaunchKernelGGL(gdn::gdn_prefill_scanw_kernel, grid, bw, 0, st, sa);
-            else if (sa.jobs && nw4)
-                hipLaunchKernelGGL(gdn::gdn_prefill_scan4_kernel<true>, grid, b4, 0, st, sa);
-            else if (sa.jobs)
-                hipLaunchKernelGGL(gdn::gdn_prefill_scan8_kernel<true>, grid, b8, 0, st, sa);
-            else if (nw4)
-                hipLaunchKernelGGL(gdn::gdn_prefill_scan4_kernel<false>, grid, b4, 0, st, sa);
-            else
-                hipLaunchKernelGGL(gdn::gdn_prefill_scan8_kernel<false>, grid, b8, 0, st, sa);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), 0, st, sa);
             return gdn_check_launch("gdn_prefill_scan_kernel");
         };
+        // one pass over the segment jobs, as many as `units`: the grid holds every form that a
+        // job count may call for
+        auto pass = [&](int64_t units) {
+            const int64_t groups = units * HQK, g4 = std::min<int64_t>(units, gdn::kPairs4 / HV) * HQK;
+            return launch(gdn::gdn_prefill_scan_any_kernel<true>, units,
+                          std::max({blocks_of(groups, 1), blocks_of(g4, 2),
+                                    blocks_of(std::min<int64_t>(groups, sa.split_groups), 4)}), 512);
+        };
+        const int64_t groups = (int64_t)N * HQK;
         if (G > 1) {
             // pass A: segment 0 of every sequence and both state maps of the middle segments
             sa.jobs = pa.jobs;
             sa.job_first = 0;
             sa.njob_idx = 1;
-            rc = scan(L.capA, L.capA * HV <= 128);
+            rc = pass(L.capA);
             if (rc)
                 return rc;
             // pass C: outputs of segments 1 .. G - 1, each chaining its entering state first;
             // the last segment's final state is new_state
             sa.job_first = (int)L.capA;
             sa.njob_idx = 2;
-            rc = scan(c4_only ? L.capC : pa.seg_c4, true);
-            if (rc == 0 && !c4_only) {
-                sa.njob_idx = 3;
-                rc = scan(L.capC, false);
-            }
+            rc = pass(L.capC);
         } else if (whole_dual) {
-            sa.ngroups = N * HQK;  // at most 256 (sequence, v-head) pairs
-            const unsigned blocks = 8 * 2 * ratio * ((sa.ngroups + 7) / 8);
-            hipLaunchKernelGGL(gdn::gdn_prefill_scan_any_kernel, dim3(blocks), dim3(512), 0, st, sa);
-            rc = gdn_check_launch("gdn_prefill_scan_any_kernel");
+            rc = launch(gdn::gdn_prefill_scan_any_kernel<false>, N, blocks_of(groups, 2), 512);
         } else if (wide) {
             sa.njob_idx = 6;
-            rc = scan(N, false, true);
+            rc = launch(gdn::gdn_prefill_scanw_kernel, N, blocks_of(groups, 1), 256);
             if (rc == 0) {
-                sa.njob_idx = 5;
-                const int64_t cus = num_cus(st);  // one workgroup per CU, at least one per queue
-                hipLaunchKernelGGL(gdn::gdn_prefill_scan8q_kernel,
-                                   dim3((unsigned)(8 * std::max<int64_t>(cus / 8, 1))), dim3(512), 0, st, sa);
-                rc = gdn_check_launch("gdn_prefill_scan8q_kernel");
+                sa.njob_idx = 5;  // one workgroup per CU, at least one per queue
+                rc = launch(gdn::gdn_prefill_scan8q_kernel, N, 8 * std::max<int64_t>(cus / 8, 1), 512);
             }
+        } else if (nw4) {
+            rc = launch(gdn::gdn_prefill_scan4_kernel, N, blocks_of(groups, groups <= sa.split_groups ? 4 : 2), 320);
         } else {
-            rc = scan(N, nw4);
+            rc = launch(gdn::gdn_prefill_scan8_kernel, N, blocks_of(groups, 1), 512);
         }
         if (rc)
             return rc;

@@ -122,9 +122,6 @@ __device__ __forceinline__ void self_plan(const PrepArgs &p, PrepSmem<VH> &sm, i
         if (l == 0) {
             q.seq_chunk0[q.N] = sm.s_total;
             q.header[0] = sm.s_total;
-            // without segments every sequence is a whole job of the one scan launch
-            q.header[1] = q.header[3] = 0;
-            q.header[2] = q.N;
         }
         if (q.seg_G >= 3)  // every lane of the wave takes part
             plan_jobs(q, order, sm.s_first, sm.s_t0, lens, l);

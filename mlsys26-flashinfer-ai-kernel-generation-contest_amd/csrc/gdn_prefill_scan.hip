@@ -739,33 +739,26 @@ __device__ __forceinline__ const ScanArgs &fresh_kernel_args()
 // Measured on MI355X, bit-identical against one segment body for every job: the qk4_v8
 // prefills of 8 sequences (all whole, or mixed with cut ones) 44.4 -> 40.9 and 54.9 -> 49.9
 // us; 1 x 4096 at 32 v-heads 98.4 -> 91.9 us.
-template <int NW, bool SEG>
-__device__ __forceinline__ void scan_kernel_body(const ScanArgs &p, ScanBuf<NW> &BA,
-                                                 ScanBuf<NW> &BB)
+template <int NW>
+__device__ __forceinline__ void seg_bodies(const ScanJob &job, ScanBuf<NW> &BA, ScanBuf<NW> &BB)
 {
-    ScanJob job;
-    if (!scan_job<NW, SEG>(p, job, blockIdx.x))
-        return;
-    if constexpr (SEG) {
-        if (job.kind == kJobFirst && job.q < 0 && job.cb == 0) {
-            scan_body<NW, false, 1>(fresh_kernel_args(), job, BA, BB);
-        } else if (job.kind == kJobFirst || job.kind == kJobResume) {
-            scan_body<NW, true, 0, 1>(fresh_kernel_args(), job, BA, BB);
-        } else if (job.kind == kJobZero) {
-            scan_body<NW, true, 0, 0>(fresh_kernel_args(), job, BA, BB);
-        } else {
-            scan_body<NW, true, 0, 2>(fresh_kernel_args(), job, BA, BB);
-        }
-    } else {
-        scan_body<NW, SEG>(p, job, BA, BB);
-    }
+    if (job.kind == kJobFirst && job.q < 0 && job.cb == 0)
+        scan_body<NW, false, 1>(fresh_kernel_args(), job, BA, BB);
+    else if (job.kind == kJobFirst || job.kind == kJobResume)
+        scan_body<NW, true, 0, 1>(fresh_kernel_args(), job, BA, BB);
+    else if (job.kind == kJobZero)
+        scan_body<NW, true, 0, 0>(fresh_kernel_args(), job, BA, BB);
+    else
+        scan_body<NW, true, 0, 2>(fresh_kernel_args(), job, BA, BB);
 }
 
-template <bool SEG>
+// Whole sequences, 8 waves: one workgroup per (sequence, v-head).
 __global__ __launch_bounds__(512) void gdn_prefill_scan8_kernel(ScanArgs p)
 {
     __shared__ ScanBuf<8> bufA, bufB;
-    scan_kernel_body<8, SEG>(p, bufA, bufB);
+    ScanJob job;
+    if (scan_job<8, false>(p, job, blockIdx.x, kAllJobs))
+        scan_body<8, false>(p, job, bufA, bufB);
 }
 
 // The 8-wave whole-sequence scan behind the wide one (choose_wide, gdn_prefill.h): one workgroup
@@ -783,7 +776,7 @@ __global__ __launch_bounds__(512) void gdn_prefill_scan8q_kernel(ScanArgs p)
     for (;;) {
         ScanJob job;
         // (a slot past the last job ends the workgroup: its queue is handed out)
-        if (slot > (0x7fffffff >> 3) || !scan_job<8, false>(p, job, 8 * slot + xcd))
+        if (slot > (0x7fffffff >> 3) || !scan_job<8, false>(p, job, 8 * slot + xcd, p.header[p.njob_idx]))
             return;
         int next = -1;  // thread 0: the next slot, pulled during the job's last chunk
         scan_body<8, false, 2>(fresh_kernel_args(), job, bufA, bufB, [&] {
@@ -798,68 +791,85 @@ __global__ __launch_bounds__(512) void gdn_prefill_scan8q_kernel(ScanArgs p)
     }
 }
 
-// LDS of the 4-wave scan kernels: the 64-row bodies' two chunk buffers or the column-split
-// bodies' buffers.
-union Scan4Lds {
-    struct {
-        ScanBuf<4> a, b;
-    } s4;
-    SplitLds sp;
+// LDS of a kernel that holds several kinds of body. The two chunk buffers are objects of their
+// own: the compiler then sees that copies in flight to one do not alias reads of the other, and
+// adds no wait for them.
+union ScanLdsA {
+    ScanBuf<8> s8;
+    ScanBuf<4> s4;
+    SplitLdsA sp;
+};
+union ScanLdsB {
+    ScanBuf<8> s8;
+    ScanBuf<4> s4;
+    SplitLdsB sp;
 };
 
-// The grid holds at most one workgroup per CU. When four workgroups per (job, v-head) fit it,
-// the column-split bodies take the jobs (32 state rows each), else the 64-row bodies (two).
-template <bool SEG>
+// Whole sequences, 4 waves and the copy wave: 64 state rows per workgroup, or 32 on the
+// column-split body where four workgroups per (sequence, v-head) find a CU each.
 __global__ __launch_bounds__(320) void gdn_prefill_scan4_kernel(ScanArgs p)
 {
-    __shared__ Scan4Lds lds;
-    const int avail = (int)(gridDim.x / (32u * p.ratio)) * 8;  // q/k head groups of four per v-head
-    const int groups = SEG ? p.header[p.njob_idx] * p.HQK : p.ngroups;
-    if (groups > avail) {
-        scan_kernel_body<4, SEG>(p, lds.s4.a, lds.s4.b);
-        return;
-    }
+    __shared__ ScanLdsA a;
+    __shared__ ScanLdsB b;
     ScanJob job;
-    if (!scan_job<2, SEG>(p, job, blockIdx.x))
-        return;
-    if constexpr (SEG) {
-        if (job.kind == kJobFirst && job.q < 0 && job.cb == 0)
-            split_body<false, 1, 1>(fresh_kernel_args(), job, lds.sp);
-        else if (job.kind == kJobFirst || job.kind == kJobResume)
-            split_body<true, 0, 1>(fresh_kernel_args(), job, lds.sp);
-        else if (job.kind == kJobZero)
-            split_body<true, 0, 0>(fresh_kernel_args(), job, lds.sp);
-        else
-            split_body<true, 0, 2>(fresh_kernel_args(), job, lds.sp);
-    } else {
-        split_body<false, 0, 1>(fresh_kernel_args(), job, lds.sp);
+    if (p.ngroups <= p.split_groups) {
+        if (scan_job<2, false>(p, job, blockIdx.x, kAllJobs))
+            split_body<false, 0, 1>(fresh_kernel_args(), job, a.sp, b.sp);
+    } else if (scan_job<4, false>(p, job, blockIdx.x, kAllJobs)) {
+        scan_body<4, false>(p, job, a.s4, b.s4);
     }
 }
 
-// Whole sequences at the planner's choice of width, in one launch: 4 waves and the copy wave (the
-// other three leave at once), two workgroups per (sequence, v-head), for header[4] sequences, or
-// 8 waves and one workgroup for header[5] of them; one of the two counts is zero. A launch for
-// each width left one of them without a job: 6 sequences of 80 to 180 tokens at 32 v-heads 27.0
-// -> 25.3 us, 20 of 400 at 8 43.2 -> 41.6, 32 of 64 to 1024 at 8 78.0 -> 76.4.
+// The planner's choice of width, in one launch: 8 waves per workgroup and one per (job, v-head),
+// or 4 waves and the copy wave (the other three leave at once) and two or four workgroups per
+// (job, v-head). SEG: segment jobs, at the width their number calls for; otherwise whole
+// sequences, all of them in the 4-wave form (header[4] of them) or the 8-wave form (header[5]).
+// Where the number of jobs is known to the device alone, a launch for each width left one of
+// them without a job, at 1.7 us: 6 sequences of 80 to 180 tokens at 32 v-heads 27.0 -> 25.3 us,
+// 20 of 400 at 8 43.2 -> 41.6, 32 of 64 to 1024 at 8 78.0 -> 76.4.
+template <bool SEG>
 __global__ __launch_bounds__(512) void gdn_prefill_scan_any_kernel(ScanArgs p)
 {
-    __shared__ ScanBuf<8> bufA, bufB;
+    __shared__ ScanLdsA a;
+    __shared__ ScanLdsB b;
     ScanJob job;
-    const int n4 = p.header[4], n8 = p.header[5];
-    if (n4 > 0) {
-        // (a scalar branch: the three waves end here, and barriers count those that are left)
-        if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) > 4)
+    int njob = p.header[SEG ? p.njob_idx : 4];
+    const bool four = SEG ? njob * p.HV <= kPairs4 : njob > 0;
+    if (!SEG && !four)
+        njob = p.header[5];
+    if (!four) {
+        if (!scan_job<8, SEG>(p, job, blockIdx.x, njob))
             return;
-        if (scan_job<4, false>(p, job, blockIdx.x))
-            scan_body<4, false, 3>(fresh_kernel_args(), job, (ScanBuf<4> &)bufA, (ScanBuf<4> &)bufB);
-    } else if (n8 > 0 && scan_job<8, false>(p, job, blockIdx.x)) {
-        scan_body<8, false, 3>(fresh_kernel_args(), job, bufA, bufB);
+        if constexpr (SEG)
+            seg_bodies<8>(job, a.s8, b.s8);
+        else
+            scan_body<8, false, 3>(fresh_kernel_args(), job, a.s8, b.s8);
+        return;
+    }
+    // (a scalar branch: the three waves end here, and barriers count those that are left)
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) > 4)
+        return;
+    if constexpr (SEG) {
+        if (njob * p.HQK <= p.split_groups) {
+            if (!scan_job<2, true>(p, job, blockIdx.x, njob))
+                return;
+            if (job.kind == kJobFirst && job.q < 0 && job.cb == 0)
+                split_body<false, 1, 1>(fresh_kernel_args(), job, a.sp, b.sp);
+            else if (job.kind == kJobFirst || job.kind == kJobResume)
+                split_body<true, 0, 1>(fresh_kernel_args(), job, a.sp, b.sp);
+            else if (job.kind == kJobZero)
+                split_body<true, 0, 0>(fresh_kernel_args(), job, a.sp, b.sp);
+            else
+                split_body<true, 0, 2>(fresh_kernel_args(), job, a.sp, b.sp);
+        } else if (scan_job<4, true>(p, job, blockIdx.x, njob)) {
+            seg_bodies<4>(job, a.s4, b.s4);
+        }
+    } else if (scan_job<4, false>(p, job, blockIdx.x, njob)) {
+        scan_body<4, false, 3>(fresh_kernel_args(), job, a.s4, b.s4);
     }
 }
 
-template __global__ void gdn_prefill_scan8_kernel<false>(ScanArgs p);
-template __global__ void gdn_prefill_scan8_kernel<true>(ScanArgs p);
-template __global__ void gdn_prefill_scan4_kernel<false>(ScanArgs p);
-template __global__ void gdn_prefill_scan4_kernel<true>(ScanArgs p);
+template __global__ void gdn_prefill_scan_any_kernel<false>(ScanArgs p);
+template __global__ void gdn_prefill_scan_any_kernel<true>(ScanArgs p);
 
 }  // namespace gdn

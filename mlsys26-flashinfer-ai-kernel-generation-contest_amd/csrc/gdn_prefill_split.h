@@ -25,10 +25,14 @@ struct SplitExch {
     u32x4 U[2][64];        // U (bf16) of tokens 0 .. 31
 };
 
-struct SplitLds {
-    SplitBuf a, b;
+// The bodies' LDS, in two parts that overlay the 64-row and 8-wave bodies' two chunk buffers
+struct SplitLdsA {
+    SplitBuf buf;
     SplitExch e;
-    u32x4 ml[kMtUnits];  // chain steps: the low half of M^T (the high half is in b)
+};
+struct SplitLdsB {
+    SplitBuf buf;
+    u32x4 ml[kMtUnits];  // chain steps: the low half of M^T (the high half is in buf)
 };
 
 // Wave (rg, hc) owns state rows v0 + 16 rg .. + 15, columns 64 hc .. + 63, and finishes the
@@ -47,10 +51,11 @@ struct SplitLds {
 // 300 at 32 19.95 -> 18.6, 1 x 1024 at 8 32.3 -> 29.6, 8 of 64 to 1024 at 8 39.7 -> 37.8. Two waves of this kind per SIMD (64 rows
 // per workgroup) were slower than one 64-row body: 8 sequences of 64 to 1024 44 -> 51 us.
 template <bool SEG, int INST, int OUTS>
-__device__ __forceinline__ void split_body(const ScanArgs &p, const ScanJob &job, SplitLds &lds)
+__device__ __forceinline__ void split_body(const ScanArgs &p, const ScanJob &job, SplitLdsA &la_,
+                                           SplitLdsB &lb_)
 {
-    SplitBuf &BA = lds.a, &BB = lds.b;
-    SplitExch &E = lds.e;
+    SplitBuf &BA = la_.buf, &BB = lb_.buf;
+    SplitExch &E = la_.e;
     constexpr bool kOut = OUTS == 1;
     const int grp = job.grp, wi = job.wi, n = job.n, tok0 = job.tok0, len = job.len,
               c0 = job.c0, kind = SEG ? job.kind : kJobFirst, cb = SEG ? job.cb : 0,
@@ -176,7 +181,7 @@ __device__ __forceinline__ void split_body(const ScanArgs &p, const ScanJob &job
     // own area) and loads R.
     const bool chain = SEG && steps > 0;
     static_assert(sizeof(SplitBuf) >= (kMtUnits + 2 * 512) * 16, "M^T hi and the exchanged state must fit");
-    u32x4 *mh = (u32x4 *)&BB, *ml = lds.ml;
+    u32x4 *mh = (u32x4 *)&BB, *ml = lb_.ml;
     auto issue_m = [&](int qs) {
         const auto rs = rsrc((const char *)(p.seg_mt + ((int64_t)qs * p.HV + h) * kSlotFloats), 2 * kMtUnits * 16);
 #pragma unroll
@@ -499,8 +504,8 @@ __device__ __forceinline__ void split_body(const ScanArgs &p, const ScanJob &job
         // This wave holds rows k = v0w .. + 15 of M_s for columns j = 64 hc .. + 63: k-chunks
         // cu0 and cu0 + 1 of those rows of M_s^T. Transposed through a per-wave LDS stage
         // (fp32, row j at 64 j bytes) in the M^T area, each unit split into bf16 hi and lo.
-        float *stg = (float *)lds.ml + 1024 * w;
-        static_assert(sizeof(lds.ml) >= 4 * 1024 * 4, "stage must fit");
+        float *stg = (float *)lb_.ml + 1024 * w;
+        static_assert(sizeof(lb_.ml) >= 4 * 1024 * 4, "stage must fit");
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll

@@ -46,7 +46,7 @@ gdn_prefill_scanw_kernel(ScanArgs p)
     // reads of another, and adds no wait for it)
     __shared__ u32x4 K0[kC * 16], K1[kC * 16], Q[kC * 16], V[kC * 16], T[704], P[320];
     ScanJob job;
-    if (!scan_job<8, false>(p, job, blockIdx.x))
+    if (!scan_job<8, false>(p, job, blockIdx.x, p.header[p.njob_idx]))
         return;
     const int n = job.n, tok0 = job.tok0, len = job.len, c0 = job.c0;
     const int g = job.grp % p.HQK, h = g * p.ratio + job.wi;

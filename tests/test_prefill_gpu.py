@@ -339,6 +339,7 @@ def _run_with_header(dev, inp, label, ints=16):
     ns = torch.empty((len(inp.seqlens), hv, 128, 128), dtype=torch.float32, device=dev)
     P, _, _, copy_back, keep, stream = _prefill_marshal(*g.args(), out, ns)
     assert not copy_back
+    keep[-1][:4 * ints].zero_()
     print(f"[{label}] launching", flush=True)
     rc = _lib.load().gdn_prefill_launch(ctypes.byref(P), ctypes.c_void_p(stream.cuda_stream))
     assert rc == 0, _lib.load().gdn_last_error()
@@ -408,67 +409,49 @@ def test_prefill_segments_mixed(dev, lens, hqk, hv):
                              state_std=0.05), f"segments lens={lens}")
 
 
-@pytest.mark.parametrize("lens,plan", [
-    (varlen_lengths(8, seed=7), (0, 8, 0)),  # 12, 11, 11, 8, 8, 7, 5, 2 chunks: no cut pays off
-    ([4096, 700, 650], (9, 7, 0)),           # 64 chunks in 6 segments; 11-chunk ones whole in C
-    ([3000, 200, 150, 100], (10, 4, 0)),     # 47 chunks in 5 segments; the short ones whole in A
-    # ten sequences: pass C launched with 4 and with 8 waves. 10-12 chunks each: nothing is
-    # cut, and the ten whole jobs fit the 4-wave launch
-    ([720, 700, 705, 690, 680, 660, 650, 640, 600, 710], (0, 10, 0)),
-    # 44-50 chunks each: all cut in 3 segments, 20 resumed segments for the 8-wave launch
-    ([3000, 2900, 3100, 2950, 3050, 2800, 3200, 2850, 3150, 2990], (30, 0, 20)),
+@pytest.mark.parametrize("lens,hqk,hv,plan", [
+    ([4096, 700, 650], 4, 8, (9, 7)),           # 64 chunks in 6 segments; 11-chunk ones whole in C
+    ([3000, 200, 150, 100], 4, 8, (10, 4)),     # 47 chunks in 5 segments; the short ones whole in A
+    # offered segments, none taken: equal lengths run whole in pass C, 4 and 10 jobs
+    ([650, 640, 600, 655], 4, 8, (0, 4)),
+    ([720, 700, 705, 690, 680, 660, 650, 640, 600, 710], 4, 8, (0, 10)),
+    ([2500, 2400], 16, 32, (0, 2)),
+    # a long prompt beside short ones
+    ([1980, 20], 4, 8, (12, 6)),
+    ([2400, 20, 20, 20], 4, 8, (10, 4)),
+    ([6000, 100, 100, 100, 100, 100], 4, 8, (10, 3)),
+    ([4000] + [20] * 11, 2, 4, (16, 3)),
+    # all cut: 7 segment jobs each in pass A (224 pairs), 16 resumed segments in pass C
+    ([8000, 7800, 7700, 7900], 4, 8, (28, 16)),
+    ([8000, 0, 7800], 8, 16, (11, 6)),
+    # ten of 44-50 chunks: cut in 3 both passes would need 8 waves and lose
+    ([3000, 2900, 3100, 2950, 3050, 2800, 3200, 2850, 3150, 2990], 4, 8, (0, 10)),
+    (varlen_lengths(8, seed=7), 4, 8, (0, 0)),  # 3-12 chunks: not offered
 ])
-def test_prefill_segment_planner(dev, lens, plan):
-    """Segment plans on few sequences (qk4_v8 heads; mild decay, so every chained state
-    carries into the next segment). Sequences of similar length all run whole in pass C
-    with pass A empty; a long sequence is cut into segments while the short ones run whole
-    in pass C beside its resumed segments, or in pass A beside its segment 0 and state maps.
-    Each segment kernel then runs every body it holds (whole sequence, segment with
-    outputs, both state maps). The job counts the planner wrote (workspace header: pass A,
-    pass C in the 4-wave launch, pass C in the 8-wave launch) name the plan taken."""
-    from gdn_hip import _lib
-    from gdn_hip.api import _prefill_marshal
-    inp = prefill_inputs(lens, hqk=4, hv=8, seed=59, with_state=True, gates="mild",
+def test_prefill_segment_planner(dev, lens, hqk, hv, plan):
+    """Segment plans on few sequences (mild decay, so every chained state carries into the next
+    segment). Sequences of similar length all run whole in pass C with pass A empty; a long
+    sequence is cut into segments while the short ones run whole in pass C beside its resumed
+    segments, or in pass A beside its segment 0 and state maps. The one kernel of both passes
+    then runs every body it holds (whole sequence, segment with outputs, both state maps) at
+    every width (column split up to 64 (job, v-head) pairs, 4 waves up to 128, 8 above). The job
+    counts the planner wrote (workspace header, cleared before: pass A, pass C) name the plan;
+    a call that is not offered segments leaves both zero."""
+    inp = prefill_inputs(lens, hqk=hqk, hv=hv, seed=59, with_state=True, gates="mild",
                          state_std=0.05)
-    ref_out, ref_ns = _oracle(inp)
-    g = inp.to(dev)
-    out = torch.empty((g.q.shape[0], 8, 128), dtype=torch.bfloat16, device=dev)
-    ns = torch.empty((len(lens), 8, 128, 128), dtype=torch.float32, device=dev)
-    P, _, _, copy_back, keep, stream = _prefill_marshal(*g.args(), out, ns)
-    assert not copy_back
-    rc = _lib.load().gdn_prefill_launch(ctypes.byref(P), ctypes.c_void_p(stream.cuda_stream))
-    assert rc == 0, _lib.load().gdn_last_error()
-    torch.cuda.synchronize()
-    header = keep[-1][:16].view(torch.int32).cpu().tolist()
-    print(f"[planner {lens[:3]}] pass A jobs {header[1]}, pass C jobs {header[2]} (4 waves) "
-          f"{header[3]} (8 waves)", flush=True)
-    assert (header[1], header[2], header[3]) == plan
-    _check(out, ns, ref_out, ref_ns, f"planner {plan}")
+    header = _run_with_header(dev, inp, f"planner {lens[:3]} x {hv}")
+    assert (header[1], header[2]) == plan
 
 
 @pytest.mark.parametrize("n,seed,use4", [(20, 4, True), (32, 6, False)])
 def test_prefill_whole_scan_choice(dev, n, seed, use4):
-    """Whole sequences with 129 to 256 (sequence, v-head) pairs: both scans are launched and
-    the prep kernel gives the sequences to the 4-wave one when its load per CU stays below
-    the longest sequence (20 qk4_v8 sequences), else to the 8-wave one (32 sequences). The
+    """Whole sequences with 129 to 256 (sequence, v-head) pairs: the prep kernel has them scanned
+    by 4 waves when neither the mean load per CU nor the two jobs that meet on the CU filled last
+    exceed 1.25 times the longest sequence (20 qk4_v8 sequences), else by 8 (32 sequences). The
     workspace header holds the counts (4-wave, 8-wave); the results hold the oracle bar."""
-    from gdn_hip import _lib
-    from gdn_hip.api import _prefill_marshal
-    lens = varlen_lengths(n, seed=seed)
-    inp = prefill_inputs(lens, hqk=4, hv=8, seed=seed, with_state=True)
-    ref_out, ref_ns = _oracle(inp)
-    g = inp.to(dev)
-    out = torch.empty((g.q.shape[0], 8, 128), dtype=torch.bfloat16, device=dev)
-    ns = torch.empty((n, 8, 128, 128), dtype=torch.float32, device=dev)
-    P, _, _, copy_back, keep, stream = _prefill_marshal(*g.args(), out, ns)
-    assert not copy_back
-    rc = _lib.load().gdn_prefill_launch(ctypes.byref(P), ctypes.c_void_p(stream.cuda_stream))
-    assert rc == 0, _lib.load().gdn_last_error()
-    torch.cuda.synchronize()
-    header = keep[-1][:32].view(torch.int32).cpu().tolist()
-    print(f"[whole scan choice N={n}] 4-wave {header[4]}, 8-wave {header[5]}", flush=True)
+    inp = prefill_inputs(varlen_lengths(n, seed=seed), hqk=4, hv=8, seed=seed, with_state=True)
+    header = _run_with_header(dev, inp, f"whole scan choice N={n}")
     assert (header[4], header[5]) == ((n, 0) if use4 else (0, n))
-    _check(out, ns, ref_out, ref_ns, f"whole scan choice N={n}")
 
 
 @pytest.mark.parametrize("seed", range(6))
