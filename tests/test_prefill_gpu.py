@@ -289,9 +289,9 @@ def test_prefill_matches_exact_fixture(dev):
 
 @pytest.mark.parametrize("nseq", [64, 65, 255, 300, 600])
 def test_prefill_many_sequences(dev, nseq):
-    """Many short and empty sequences. Up to 64 the prep kernel plans for itself (one
-    sequence per lane); from 65 the planning kernel's chunk table and longest-first order
-    (its sort covers up to 512 sequences) drive prep and scan."""
+    """Many short and empty sequences. Up to 126 the prep kernel plans for itself (one
+    sequence per lane up to 64, two above); from 127 the planning kernel's chunk table and
+    longest-first order (its sort covers up to 512 sequences) drive prep and scan."""
     g = torch.Generator().manual_seed(nseq)
     lens = [int(x) for x in torch.randint(0, 90, (nseq,), generator=g)]
     _run(dev, prefill_inputs(lens, hqk=4, hv=8, seed=nseq, with_state=True), f"N={nseq}")
@@ -328,15 +328,17 @@ def test_prefill_wide_scan(dev, lens, hqk, hv, state, gates):
                              gates=gates), f"wide scan {len(lens)} x {hv}")
 
 
-def _run_with_header(dev, inp, label, ints=16):
+def _run_with_header(dev, inp, label, ints=16, inplace=False):
     """One prefill through the C entry point against the oracle; returns the first ints of
-    the workspace header, where the planner leaves its job counts."""
+    the workspace header, where the planner leaves its job counts (cleared before: a call that
+    plans none leaves zeros)."""
     from gdn_hip.api import _prefill_marshal
     ref_out, ref_ns = _oracle(inp)
     g = inp.to(dev)
     hv = g.v.shape[1]
     out = torch.empty(g.v.shape, dtype=torch.bfloat16, device=dev)
-    ns = torch.empty((len(inp.seqlens), hv, 128, 128), dtype=torch.float32, device=dev)
+    ns = g.state if inplace else torch.empty((len(inp.seqlens), hv, 128, 128),
+                                             dtype=torch.float32, device=dev)
     P, _, _, copy_back, keep, stream = _prefill_marshal(*g.args(), out, ns)
     assert not copy_back
     keep[-1][:4 * ints].zero_()
@@ -368,11 +370,59 @@ def test_prefill_wide_scan_choice(dev, lens, hqk, hv, wide):
     assert (header[5], header[6]) == ((0, n) if wide else (n, 0))
 
 
+@pytest.mark.parametrize("skewed", [False, True])
+def test_prefill_wide_scan_layouts(dev, skewed):
+    """768 pairs, in the wide scan and (one long sequence) in the queued 8-wave scan behind it:
+    q / k / v as views of a fused projection, the output a view of a wider tensor, the state
+    strided and updated in place, tokens before the first and after the last sequence."""
+    lens = [1 + (37 * i) % 130 for i in range(96)]
+    if skewed:
+        lens[40] = 1900
+    inp = prefill_inputs(lens, hqk=4, hv=8, seed=17, with_state=True, gates="mild", pad_tokens=9)
+    inp.cu_seqlens = inp.cu_seqlens + 4
+    ref_out, ref_ns = _oracle(inp)
+    g = inp.to(dev)
+    T = g.q.shape[0]
+    qkv = torch.cat([g.q, g.k, g.v], dim=1)
+    big = torch.full((T, 12, 128), 7.0, dtype=torch.bfloat16, device=dev)
+    st = torch.full((96, 11, 128, 132), 3.0, dtype=torch.float32, device=dev)
+    st[:, 2:10, :, :128] = g.state
+    state, out = st[:, 2:10, :, :128], big[:, 3:11]
+    print(f"[wide layouts skewed={skewed}] launching", flush=True)
+    o, ns = gdn_prefill(qkv[:, :4], qkv[:, 4:8], qkv[:, 8:], state, g.A_log, g.a, g.dt_bias, g.b,
+                        g.cu_seqlens, g.scale, output=out, new_state=state)
+    torch.cuda.synchronize()
+    assert o.data_ptr() == out.data_ptr() and ns.data_ptr() == state.data_ptr()
+    _check(o, ns, ref_out, ref_ns, f"wide layouts skewed={skewed}")
+    assert not out[:4].any() and not out[-5:].any()
+    assert torch.all(big[:, :3] == 7) and torch.all(big[:, 11:] == 7)
+    st[:, 2:10, :, :128] = 3.0
+    assert torch.all(st == 3)
+
+
+@pytest.mark.parametrize("cu_dtype", [torch.int32, torch.int64])
+def test_prefill_planners_agree(dev, cu_dtype):
+    """The prep kernel's own planning (126 sequences) and the plan kernel (the same and an empty
+    one) give equal bits: empty sequences, chunk edges, a first entry below 0 and last ones past
+    the end, which both clamp."""
+    lens = [(0, 1, 64, 65, 130, 20)[i % 6] for i in range(126)]
+    g = prefill_inputs(lens, hqk=2, hv=4, seed=5, with_state=True, gates="mild",
+                       cu_dtype=cu_dtype).to(dev)
+    cu = g.cu_seqlens.clone()
+    cu[0] = -7
+    cu[-3:] = g.q.shape[0] + 1000
+    rest = (g.A_log, g.a, g.dt_bias, g.b)
+    o1, s1 = gdn_prefill(g.q, g.k, g.v, g.state, *rest, cu, g.scale)
+    o2, s2 = gdn_prefill(g.q, g.k, g.v, torch.cat([g.state, g.state[:1]]), *rest,
+                         torch.cat([cu, cu[-1:]]), g.scale)
+    torch.cuda.synchronize()
+    assert torch.equal(o1, o2) and torch.equal(s1, s2[:126]) and torch.equal(s2[126], g.state[0])
+
+
 @pytest.mark.parametrize("nseq", [63, 64, 65, 125, 126, 127])
 def test_prefill_planning_limits(dev, nseq):
     """One and two planned sequences per lane, and the plan kernel above 126: empty and short
-    sequences, chunk edges, tokens before the first and after the last, both cu_seqlens types;
-    every path gives the same chunk numbering, so equal inputs give equal bits."""
+    sequences, chunk edges, tokens before the first and after the last, both cu_seqlens types."""
     lens = [(0, 1, 64, 65, 130, 20)[i % 6] for i in range(nseq)]
     inp = prefill_inputs(lens, hqk=2, hv=4, seed=nseq, with_state=True, gates="mild",
                          cu_dtype=torch.int64 if nseq % 2 else torch.int32, pad_tokens=7)
@@ -400,13 +450,17 @@ def test_prefill_segments_long_memory(dev, gates):
          f"segments gates={gates}")
 
 
-@pytest.mark.parametrize("lens,hqk,hv", [([1500, 300], 16, 32), ([3000], 4, 8),
-                                         ([900, 0, 1400, 65], 4, 8)])
-def test_prefill_segments_mixed(dev, lens, hqk, hv):
-    """Segmented and whole sequences in one call (short ones are not split), up to eight
-    segments per sequence, empty sequences."""
-    _run(dev, prefill_inputs(lens, hqk=hqk, hv=hv, seed=43, with_state=True, gates="mild",
-                             state_std=0.05), f"segments lens={lens}")
+@pytest.mark.parametrize("lens,hqk,hv,cut", [([3000, 300], 16, 32, True), ([3000], 4, 8, True),
+                                             ([900, 0, 1400, 65], 4, 8, True),
+                                             ([1500, 300], 16, 32, False)])
+def test_prefill_segments_mixed(dev, lens, hqk, hv, cut):
+    """Segmented and whole sequences in one call (short ones are not split), up to nine
+    segments per sequence, empty sequences; and a mix that runs whole."""
+    inp = prefill_inputs(lens, hqk=hqk, hv=hv, seed=43, with_state=True, gates="mild",
+                         state_std=0.05)
+    header = _run_with_header(dev, inp, f"segments lens={lens}")
+    # a cut sequence: 3 jobs in pass A, 2 in pass C
+    assert header[1] >= 3 and header[2] >= 2 if cut else header[1] == 0
 
 
 @pytest.mark.parametrize("lens,hqk,hv,plan", [
@@ -454,41 +508,53 @@ def test_prefill_whole_scan_choice(dev, n, seed, use4):
     assert (header[4], header[5]) == ((n, 0) if use4 else (0, n))
 
 
-@pytest.mark.parametrize("seed", range(6))
-def test_prefill_segment_planner_random(dev, seed):
+@pytest.mark.parametrize("seed,plan", [(0, "cut"), (1, "cut"), (2, "none"), (3, "whole"),
+                                       (4, "cut"), (5, "cut"), (8, "cut"), (12, "whole"),
+                                       (14, "cut")])
+def test_prefill_segment_planner_random(dev, seed, plan):
     """Random mixes in the segment regime (2 to 10 sequences, qk4_v8 heads, N HV 3 <= 256):
     long sequences that may be cut beside short and empty ones, so plans mix cut sequences,
     whole jobs in either pass and the all-whole plan; mild decay keeps every chained state
-    significant."""
+    significant. The job counts say which kind of plan each mix took ("none": too short to be
+    offered segments)."""
     rng = np.random.default_rng(1000 + seed)
     n = int(rng.integers(2, 11))
     lens = [int(rng.choice([rng.integers(0, 3), rng.integers(1, 400), rng.integers(400, 1400),
                              rng.integers(1400, 3200)], p=[0.1, 0.35, 0.35, 0.2]))
             for _ in range(n)]
-    _run(dev, prefill_inputs(lens, hqk=4, hv=8, seed=70 + seed, with_state=True, gates="mild",
-                             state_std=0.05), f"planner mix {seed} lens={lens}")
+    header = _run_with_header(dev, prefill_inputs(lens, hqk=4, hv=8, seed=70 + seed, with_state=True,
+                                                  gates="mild", state_std=0.05),
+                              f"planner mix {seed} lens={lens}")
+    jobs = header[1:3]
+    if plan == "cut":
+        assert jobs[0] >= 3 and jobs[1] >= 2
+    else:
+        assert jobs == ([0, n] if plan == "whole" else [0, 0])
 
 
-def test_prefill_long_sequences_among_many_plan_kernel(dev):
-    """Two long sequences among 68 short ones with one v-head: more than 64 sequences, so
-    the plan kernel builds the tables and every sequence is scanned whole (the job planner,
-    and with it segments, serves up to 64 sequences)."""
+@pytest.mark.parametrize("short", [68, 128])
+def test_prefill_long_sequences_among_many_plan_kernel(dev, short):
+    """Two long sequences among 68 or 128 short ones with one v-head: every sequence is scanned
+    whole (the job planner, and with it segments, serves up to 64 sequences), and above 126
+    sequences the plan kernel builds the tables."""
     rng = np.random.default_rng(77)
-    lens = [int(x) for x in rng.integers(0, 40, 68)] + [2500, 1900]
+    lens = [int(x) for x in rng.integers(0, 40, short)] + [2500, 1900]
     _run(dev, prefill_inputs(lens, hqk=1, hv=1, seed=78, with_state=True, gates="mild",
                              state_std=0.05), f"plan-kernel segments N={len(lens)}")
 
 
-def test_prefill_segments_inplace_state(dev):
+@pytest.mark.parametrize("lens,hqk,hv,cut", [([2048], 16, 32, True), ([3000, 20], 16, 32, True),
+                                             ([2048, 1100], 4, 8, True),
+                                             ([1400, 0, 1200, 900], 4, 8, True),
+                                             ([2048, 1100], 16, 32, False)])
+def test_prefill_segments_inplace_state(dev, lens, hqk, hv, cut):
     """Segmented scan with new_state aliasing state: pass A reads the initial state only in
-    segment 0's job, and only the last segment's pass-C job writes the final state."""
-    inp = prefill_inputs([2048, 1100], seed=53, with_state=True, gates="mild", state_std=0.05)
-    ref_out, ref_ns = _oracle(inp)
-    g = inp.to(dev)
-    out, ns = gdn_prefill(*g.args(), new_state=g.state)
-    torch.cuda.synchronize()
-    assert ns.data_ptr() == g.state.data_ptr()
-    _check(out, ns, ref_out, ref_ns, "segments in-place")
+    segment 0's job, and only the last segment's pass-C job writes the final state; whole
+    sequences read and write theirs in one job of either pass."""
+    inp = prefill_inputs(lens, hqk=hqk, hv=hv, seed=53, with_state=True, gates="mild",
+                         state_std=0.05)
+    header = _run_with_header(dev, inp, f"segments in-place {lens}", inplace=True)
+    assert header[1] >= 3 and header[2] >= 2 if cut else header[1] == 0
 
 
 def test_prefill_segments_match_whole_sequence_scan(dev):
@@ -537,20 +603,13 @@ def _random_case(i):
                          pad_tokens=int(rng.choice([0, 0, 3, 70])))
     if gates == "extreme":
         inp = with_extreme_gates(inp, seed=7300 + i)
-    # segments per long sequence the launcher allows (1: whole-sequence scan)
-    G = 1
-    if n and n * hv * 3 <= 256:
-        G = 3
-        while G < 8 and n * hv * (2 * G - 1) <= 256:
-            G += 1
-    return inp, f"random {i}: hqk={hqk} hv={hv} gates={gates} segments<={G} lens={lens}"
+    return inp, f"random {i}: hqk={hqk} hv={hv} gates={gates} lens={lens}"
 
 
 @pytest.mark.parametrize("i", range(10))
 def test_prefill_random_cases(dev, i):
-    """Seeded random mixes that reach the planner's and the segment scan's branches
-    (1..8 segments, balanced and equal segment lengths, short and empty sequences next
-    to long ones) under every gate regime."""
+    """Seeded random mixes of 1 to 25 sequences (short and empty ones next to long ones, whole
+    and in segments) under every gate regime."""
     inp, label = _random_case(i)
     _run(dev, inp, label)
 
