@@ -246,7 +246,7 @@ constexpr float kSegEmptyPass = 4.f;  // a pass without a job (1.7 us)
 struct PlanArgs {
     const void *cu;
     int cu64, N, T, HO, nc;  // nc: chunk-table capacity (workspace bound)
-    int32_t *header, *chunk_tok0, *chunk_len, *seq_chunk0, *seq_tok0, *seq_len;
+    int32_t *header, *chunk_tok0, *chunk_len;
     // longest-first order: seq_rank[4 r .. 4 r + 3] = {sequence, first token, length, first
     // chunk} of the r-th longest sequence (one 16-byte load per scan workgroup)
     int32_t *seq_rank;
@@ -507,7 +507,7 @@ struct ScanArgs {
     bf16_t *out;
     int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh;
     int64_t st_sn, st_sh, st_sv, ns_sn, ns_sh, ns_sv;
-    const int32_t *header, *seq_chunk0, *seq_tok0, *seq_len, *seq_rank;
+    const int32_t *header, *seq_rank;
     const char *records;
     int HQK, HV, ratio, ngroups;
     int split_groups;  // (job, q/k head) groups whose four workgroups per v-head find a CU each

@@ -72,8 +72,7 @@ int seg_count(int64_t T, int64_t N, int64_t HV)
 
 struct Layout {
     int64_t nc;
-    int64_t header, chunk_tok0, chunk_len, seq_chunk0, seq_rank, seq_tok0, seq_len, records,
-        total;
+    int64_t header, chunk_tok0, chunk_len, seq_rank, records, total;
     int G;                // segments per sequence at most (1: none)
     int64_t capA, capC;   // pass A / pass C job capacity
     int64_t jobs, seg_sin, seg_r, seg_mt;
@@ -93,14 +92,8 @@ Layout layout(int64_t T, int64_t N, int64_t HV)
     o += L.nc * 4;
     L.chunk_len = o;
     o += L.nc * 4;
-    L.seq_chunk0 = o;
-    o += (N + 1) * 4;
     L.seq_rank = (o + 15) & ~int64_t(15);
     o = L.seq_rank + N * 16;
-    L.seq_tok0 = o;
-    o += N * 4;
-    L.seq_len = o;
-    o += N * 4;
     L.records = align256(o);
     o = L.records + L.nc * HV * gdn::kRecBytes;
     L.jobs = L.seg_sin = L.seg_r = L.seg_mt = 0;
@@ -236,10 +229,7 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
     pa.header = (int32_t *)(ws + L.header);
     pa.chunk_tok0 = (int32_t *)(ws + L.chunk_tok0);
     pa.chunk_len = (int32_t *)(ws + L.chunk_len);
-    pa.seq_chunk0 = (int32_t *)(ws + L.seq_chunk0);
     pa.seq_rank = (int32_t *)(ws + L.seq_rank);
-    pa.seq_tok0 = (int32_t *)(ws + L.seq_tok0);
-    pa.seq_len = (int32_t *)(ws + L.seq_len);
     pa.out = (gdn::bf16_t *)p->output;
     pa.o_st = p->output_stride[0];
     pa.o_sh = p->output_stride[1];
@@ -361,10 +351,7 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
         sa.ns_sh = p->new_state_stride[1];
         sa.ns_sv = p->new_state_stride[2];
         sa.header = pa.header;
-        sa.seq_chunk0 = pa.seq_chunk0;
         sa.seq_rank = pa.seq_rank;
-        sa.seq_tok0 = pa.seq_tok0;
-        sa.seq_len = pa.seq_len;
         sa.records = ws + L.records;
         sa.HQK = HQK;
         sa.HV = HV;

@@ -34,8 +34,6 @@ __global__ __launch_bounds__(256) void gdn_prefill_plan_kernel(PlanArgs p)
                 ln = (int)(b - a);
                 nck = (ln + kC - 1) / kC;
                 cmax = fmaxf(cmax, (float)nck);
-                p.seq_tok0[n] = t0;
-                p.seq_len[n] = ln;
                 if (n < kPlanSortMax)
                     s_nck[n] = nck;
             }
@@ -49,7 +47,6 @@ __global__ __launch_bounds__(256) void gdn_prefill_plan_kernel(PlanArgs p)
                 incl += s_wtot[w2];
             const int64_t first = s_carry + incl - nck;
             if (n < p.N) {
-                p.seq_chunk0[n] = (int32_t)(first < p.nc ? first : p.nc);
                 if (par) {
                     s_first[n] = (int32_t)(first < p.nc ? first : p.nc);
                     s_end[n] = (int32_t)(first + nck < p.nc ? first + nck : p.nc);
@@ -72,7 +69,6 @@ __global__ __launch_bounds__(256) void gdn_prefill_plan_kernel(PlanArgs p)
         }
         if (tid == 0) {
             const int32_t total = (int32_t)(s_carry < p.nc ? s_carry : p.nc);
-            p.seq_chunk0[p.N] = total;
             p.header[0] = total;
         }
         if (p.wide_cus > 0) {

@@ -104,11 +104,7 @@ __device__ __forceinline__ void self_plan(const PrepArgs &p, PrepSmem<VH> &sm, i
         // the second K buffer is not written before the first unit's barrier
         int32_t *order = (int32_t *)sm.K[1], *lens = order + 64;
         auto put = [&](int n, int r) {
-            const int t0 = sm.s_t0[n], ln = len_of(n), first = sm.s_first[n];
-            q.seq_tok0[n] = t0;
-            q.seq_len[n] = ln;
-            q.seq_chunk0[n] = first;
-            *(int4 *)(q.seq_rank + 4 * r) = int4{n, t0, ln, first};
+            *(int4 *)(q.seq_rank + 4 * r) = int4{n, sm.s_t0[n], len_of(n), sm.s_first[n]};
         };
         if (l < q.N) {
             put(l, rank);
@@ -119,10 +115,8 @@ __device__ __forceinline__ void self_plan(const PrepArgs &p, PrepSmem<VH> &sm, i
         }
         if (64 + l < q.N)
             put(64 + l, rank1);
-        if (l == 0) {
-            q.seq_chunk0[q.N] = sm.s_total;
+        if (l == 0)
             q.header[0] = sm.s_total;
-        }
         if (q.seg_G >= 3)  // every lane of the wave takes part
             plan_jobs(q, order, sm.s_first, sm.s_t0, lens, l);
         if (q.whole_cus > 0) {
