@@ -213,15 +213,15 @@ def gdn_decode(q, k, v, state, A_log, a, dt_bias, b, scale, output=None, new_sta
     """
     if scale is None or type(scale) is float:
         fast = _lib.fast()
+        sc = 0.0 if scale is None else scale
         if fast is None:
             pass
         elif output is not None and new_state is not None:
-            if fast.decode(q, k, v, state, A_log, a, dt_bias, b, 0.0 if scale is None else scale,
-                           output, new_state, 0) == 0:
+            if fast.decode(q, k, v, state, A_log, a, dt_bias, b, sc, output, new_state, 0) == 0:
                 return output, new_state
         else:
-            r = _alloc_call(fast.decode_alloc, q, k, v, state, A_log, a, dt_bias, b,
-                            0.0 if scale is None else scale, output, new_state, 0)
+            r = _alloc_call(fast.decode_alloc, q, k, v, state, A_log, a, dt_bias, b, sc, output,
+                            new_state, 0)
             if r is not None:
                 return r
     with torch.no_grad():
@@ -449,16 +449,16 @@ def gdn_prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output=
     """
     if scale is None or type(scale) is float:
         fast = _lib.fast()
+        sc = 0.0 if scale is None else scale
         if fast is None:
             pass
         elif output is not None and new_state is not None:
-            if fast.prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens,
-                            0.0 if scale is None else scale, output, new_state,
-                            _prefill_variant) == 0:
+            if fast.prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, sc, output,
+                            new_state, _prefill_variant) == 0:
                 return output, new_state
         else:
             r = _alloc_call(fast.prefill_alloc, q, k, v, state, A_log, a, dt_bias, b, cu_seqlens,
-                            0.0 if scale is None else scale, output, new_state, _prefill_variant)
+                            sc, output, new_state, _prefill_variant)
             if r is not None:
                 return r
     with torch.no_grad():
