@@ -231,10 +231,12 @@ constexpr float kSegChainChunks = 0.9f;
 // Up to this many (job, v-head) pairs a scan runs 4 waves per workgroup, two workgroups a pair
 constexpr int kPairs4 = 128;
 
-// A scan chunk's time in k cycles (MI355X, one job per workgroup) with this many (job, v-head)
-// pairs: the column-split bodies up to 64, the 4-wave scan up to 128, the 8-wave scan (6.5 on
-// its own; 7.6 fits the best of the segment counts measured in gdn_prefill.hip). A state map's
-// chunk (no outputs) takes kSegFirstWeight of it.
+// A scan chunk's time in k cycles of 2.4 GHz (MI355X, one job per workgroup) with this many (job,
+// v-head) pairs: the column-split bodies up to 64, the 4-wave scan up to 128, the 8-wave scan. A
+// state map's chunk (no outputs) takes kSegFirstWeight of it. The 8-wave figure is that of a
+// pass on most of the chip: with 224 pairs pass A of 1 x 4096 and 1 x 8192 at 32 v-heads took 42.6
+// and 71.6 us for 14.4 and 27.6 state-map chunks and ~3 us of start, 7.9 and 7.2; on few CUs,
+// where the clock stays higher, a chunk takes 6.5.
 __host__ __device__ inline float chunk_cost(int64_t pairs)
 {
     return pairs <= 64 ? 3.6f : pairs <= kPairs4 ? 4.4f : 7.6f;

@@ -26,7 +26,7 @@ int64_t max_chunks(int64_t T, int64_t N) { return (T + kChunkH - 1) / kChunkH + 
 // Whole prefills, as many segments as pass A holds -> this rule: at 8 v-heads 1 x 4096 64.1 ->
 // 51.1 us (9 segments; 5 59.4), 1 x 8192 90.5 -> 74.8 (9), 1 x 16384 131.3 -> 128.5 (9; 12 136.0);
 // at 32 v-heads 1 x 800 33.9 -> 32.5 (whole), 1 x 1200 47.7 -> 42.1 (3), 1 x 1600 52.4 -> 48.8
-// (3), 1 x 4096 93 (5; 3 97).
+// (3), 1 x 4096 90 (5; 3 is 4 % slower).
 //
 // More sequences: only the device knows their lengths. It weighs its plan against scanning every
 // sequence whole (plan_jobs); what is decided here is whether it may cut, since a pass A without
