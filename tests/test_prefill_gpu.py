@@ -678,6 +678,41 @@ def test_prefill_in_graph(dev):
         assert torch.equal(ns, eager_ns), f"replay {r}: new_state differs"
 
 
+@pytest.mark.parametrize("lens,hqk,hv", [
+    ([1900] + [1 + (37 * i) % 130 for i in range(95)], 4, 8),  # queued 8-wave scan <-> wide
+    ([2400, 20, 20, 20], 4, 8),                                # segments <-> whole sequences
+    ([1500, 400] + [100] * 18, 4, 8),                          # 4 waves <-> 8 waves
+])
+def test_prefill_graph_replays_other_lengths(dev, lens, hqk, hv):
+    """A captured prefill replayed with the lengths of its sequences changed in cu_seqlens: the
+    planner chooses anew on every replay (its job counts and queues start from zero each time),
+    and each equals the eager call on the same lengths bit for bit."""
+    n, T = len(lens), sum(lens)
+    g = prefill_inputs(lens, hqk=hqk, hv=hv, seed=7, with_state=True, gates="mild").to(dev)
+    skewed = g.cu_seqlens.clone()
+    even = torch.tensor([T * i // n for i in range(n + 1)], dtype=torch.int32, device=dev)
+    eager = []
+    for cu in (skewed, even):
+        g.cu_seqlens.copy_(cu)
+        eager.append(gdn_prefill(*g.args()))
+    assert not torch.equal(eager[0][0], eager[1][0])
+    out, ns = torch.empty_like(eager[0][0]), torch.empty_like(eager[0][1])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        gdn_prefill(*g.args(), output=out, new_state=ns)
+    for r in range(5):
+        i = (0, 1, 1, 0, 0)[r]
+        g.cu_seqlens.copy_((skewed, even)[i])
+        out.zero_()
+        ns.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager[i][0]), f"replay {r}: output differs"
+        assert torch.equal(ns, eager[i][1]), f"replay {r}: new_state differs"
+
+
 def test_prefill_graphs_keep_their_own_workspaces(dev):
     """Two graphs captured one after the other, the second needing a larger workspace, and
     an eager call in between: each graph keeps its own workspace, so replaying the first
