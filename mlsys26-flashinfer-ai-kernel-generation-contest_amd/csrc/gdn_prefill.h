@@ -25,8 +25,9 @@
 //         fp32-valued operands on the state path (S0, R, T, U) are split into bf16
 //         hi + lo halves so the state keeps ~2^-16 relative accuracy. With few
 //         sequences, long ones are cut into segments scanned in parallel (two scan
-//         launches over job tables). With many sequences the scan runs on 32x32 tiles,
-//         32 state rows per wave and two workgroups per CU (gdn_prefill_wide.hip).
+//         launches over job tables, at the width that the plan calls for). With many
+//         sequences the scan runs on 32x32 tiles, 32 state rows per wave and two workgroups
+//         per CU (gdn_prefill_wide.hip).
 //
 // Files: gdn_prefill.h (records, layouts, argument structs, shared helpers),
 // gdn_prefill_plan.hip, gdn_prefill_prep.hip, gdn_prefill_scan.hip, gdn_prefill_split.h (a

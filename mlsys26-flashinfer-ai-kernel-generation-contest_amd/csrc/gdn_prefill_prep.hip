@@ -120,7 +120,7 @@ __device__ __forceinline__ void self_plan(const PrepArgs &p, PrepSmem<VH> &sm, i
         if (q.seg_G >= 3)  // every lane of the wave takes part
             plan_jobs(q, order, sm.s_first, sm.s_t0, lens, l);
         if (q.whole_cus > 0) {
-            // Whole sequences, both scans launched. The 8-wave scan has a CU for each (sequence,
+            // Whole sequences, either width of the scan. The 8-wave scan has a CU for each (sequence,
             // v-head) and takes the longest sequence's chunks; a chunk of the 4-wave scan is
             // 1.5 times as fast, but its twice as many workgroups share the CUs: besides the
             // longest sequence, the mean load per CU and the two jobs that meet on the CU filled

@@ -1,4 +1,4 @@
-// Column-split scan body (part of the 4-wave scan kernels): 32 state rows per workgroup, each
+// Column-split scan body (in the 4-wave scan and the segment kernel): 32 state rows per workgroup, each
 // 16-row group's work of a chunk split over two waves.
 #pragma once
 

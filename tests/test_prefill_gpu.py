@@ -615,7 +615,7 @@ def test_prefill_random_cases(dev, i):
 
 
 def test_prefill_long_sequence_64k(dev):
-    """One 65536-token sequence (1024 chunks): eight segments of ~128 chunks with their state
+    """One 65536-token sequence (1024 chunks): sixteen segments of ~64 chunks with their state
     chain, mild decay so every segment's state carries into the next."""
     inp = prefill_inputs([65536], hqk=1, hv=2, seed=97, with_state=True, gates="mild",
                          state_std=0.05)
