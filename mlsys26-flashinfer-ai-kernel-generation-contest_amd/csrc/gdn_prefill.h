@@ -534,6 +534,17 @@ struct ScanJob {
 
 constexpr int kAllJobs = 0x7fffffff;
 
+// What the planner wrote is constant in the scans: read through the constant address space, so
+// that uniform reads stay scalar loads where the compiler cannot rule out that the kernel's own
+// stores, of an earlier job say, changed it. (A vector load's wait would also wait for those
+// stores.)
+template <class V>
+__device__ __forceinline__ V plan_load(const int32_t *p)
+{
+    typedef const V __attribute__((address_space(4))) *P;
+    return *(P)(uintptr_t)p;
+}
+
 // Finds the job of workgroup pid (SEG: in the segment job table) among the first njob; false
 // when it has none.
 template <int NW, bool SEG>
@@ -575,7 +586,8 @@ __device__ __forceinline__ bool scan_job(const ScanArgs &p, ScanJob &j, int pid,
     } else {
         // ranks below ngroups / HQK = N all have an entry: load it with the count
         const int e = j.grp / p.HQK;
-        const int4 r = *(const int4 *)(p.seq_rank + 4 * e);
+        typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+        const i32x4 r = plan_load<i32x4>(p.seq_rank + 4 * e);
         if (e >= njob)
             return false;
         j.n = r.x;

@@ -54,7 +54,7 @@ __device__ __forceinline__ void scan_body(const ScanArgs &p, const ScanJob &job,
     const int h = g * p.ratio + wi / TPH;
     const int v0 = (wi % TPH) * 16 * NW;
     // records exist only for chunk ids < header[0] (see the plan kernel's clamp)
-    const int nck = min((len + kC - 1) / kC, max(p.header[0] - c0, 0));
+    const int nck = min((len + kC - 1) / kC, max(plan_load<int32_t>(p.header) - c0, 0));
     ce = min(ce, nck);
     const bool do_out = OUTS >= 0 ? OUTS == 1 : kind == kJobFirst || kind == kJobResume;
     const bool vzero = OUTS == 2 || (OUTS < 0 && kind == kJobIdent);
@@ -770,13 +770,19 @@ __global__ __launch_bounds__(512) void gdn_prefill_scan8q_kernel(ScanArgs p)
 {
     __shared__ ScanBuf<8> bufA, bufB;
     __shared__ int32_t s_slot;
-    const int xcd = blockIdx.x & 7;
+    const int xcd = blockIdx.x & 7, njob = p.header[p.njob_idx];
     int slot = blockIdx.x >> 3;
-    auto pull = [&] { return (int)(gridDim.x >> 3) + atomicAdd(p.queue + xcd, 1); };
+    // (with an address that the compiler takes for divergent: an atomic on a uniform one becomes a
+    // wave-wide sum whose result is waited for at once)
+    auto pull = [&] {
+        int none = 0;
+        asm volatile("" : "+v"(none));
+        return atomicAdd(p.queue + xcd + none, 1);
+    };
     for (;;) {
         ScanJob job;
         // (a slot past the last job ends the workgroup: its queue is handed out)
-        if (slot > (0x7fffffff >> 3) || !scan_job<8, false>(p, job, 8 * slot + xcd, p.header[p.njob_idx]))
+        if (slot > (0x7fffffff >> 3) || !scan_job<8, false>(p, job, 8 * slot + xcd, njob))
             return;
         int next = -1;  // thread 0: the next slot, pulled during the job's last chunk
         scan_body<8, false, 2>(fresh_kernel_args(), job, bufA, bufB, [&] {
@@ -784,10 +790,12 @@ __global__ __launch_bounds__(512) void gdn_prefill_scan8q_kernel(ScanArgs p)
                 next = pull();
         });
         if (threadIdx.x == 0)
-            s_slot = next >= 0 ? next : pull();  // (an empty sequence has no chunk)
-        __syncthreads();  // every wave is done with the buffers
+            s_slot = (int)(gridDim.x >> 3) + (next >= 0 ? next : pull());  // (an empty sequence has no chunk)
+        // every wave is done with the buffers; the state's stores stay in flight under the next
+        // job's first loads
+        lds_barrier_inflight();
         slot = __builtin_amdgcn_readfirstlane(s_slot);
-        __syncthreads();  // s_slot is free again
+        lds_barrier_inflight();  // s_slot is free again
     }
 }
 
