@@ -242,6 +242,16 @@ __host__ __device__ inline float chunk_cost(int64_t pairs)
 {
     return pairs <= 64 ? 3.6f : pairs <= kPairs4 ? 4.4f : 7.6f;
 }
+// The same for sequences scanned whole in a call of this many chunks x v-heads. Each of those is
+// ~64 KB of inputs, output and records; past the ~220 MB that stay in the 256 MB cache between
+// prep and scan the column-split scan's chunks wait for HBM (1 x 4096 / 8192 / 16000 at 48 v-heads:
+// 3.6, 4.1 and 4.4 k cycles; the slower scans' chunks cover it).
+constexpr float kCacheChunks = 3500.f;
+__host__ __device__ inline float whole_chunk_cost(int64_t pairs, float chunks)
+{
+    const float c = chunk_cost(pairs);
+    return pairs <= 64 && chunks > kCacheChunks ? c + 1.2f * (1.f - kCacheChunks / chunks) : c;
+}
 constexpr float kSegPassCost = 14.f;  // a second pass: its launch, state and first chunk
 constexpr float kSegEmptyPass = 4.f;  // a pass without a job (1.7 us)
 
@@ -412,7 +422,7 @@ __device__ inline void plan_jobs(const PlanArgs &p, const int32_t *order, const 
               inC = __popcll(in_c);
     const float cut = w * chunk_cost((int64_t)(p.N - inC + 2 * nmid) * p.HO) * spanA +
                       chunk_cost((int64_t)(nc + nmid + inC) * p.HO) * spanC + kSegPassCost - kSegEmptyPass;
-    const bool whole_all = nc == 0 || (p.N > 1 && chunk_cost((int64_t)p.N * p.HO) * cmax <= cut);
+    const bool whole_all = nc == 0 || (p.N > 1 && whole_chunk_cost((int64_t)p.N * p.HO, (float)p.T * p.HO / kC) * cmax <= cut);
     const bool whole = whole_all || G == 1;
     const bool wc = whole_all || ((in_c >> lane) & 1);
     // job counts -> offsets (exclusive prefix sums in rank order)
@@ -696,5 +706,12 @@ template <bool SEG>
 __global__ __launch_bounds__(512) void gdn_prefill_scan_any_kernel(ScanArgs p);
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 gdn_prefill_scanw_kernel(ScanArgs p);
+
+// ------------------------------------------------------------------------- host
+// gdn_prefill_launch; cached: with segment counts that leave the cost of a large footprint out
+// (whole_chunk_cost), which need prefill_workspace_cached() bytes instead of
+// gdn_prefill_workspace_size(): fewer where the footprint makes a sequence worth cutting.
+int prefill_launch(const gdn_prefill_params *p, void *stream, bool cached);
+int64_t prefill_workspace_cached(int64_t T, int64_t N, int64_t HV);
 
 }  // namespace gdn

@@ -26,7 +26,8 @@ int64_t max_chunks(int64_t T, int64_t N) { return (T + kChunkH - 1) / kChunkH + 
 // Whole prefills, as many segments as pass A holds -> this rule: at 8 v-heads 1 x 4096 64.1 ->
 // 51.1 us (9 segments; 5 59.4), 1 x 8192 90.5 -> 74.8 (9), 1 x 16384 131.3 -> 128.5 (9; 12 136.0);
 // at 32 v-heads 1 x 800 33.9 -> 32.5 (whole), 1 x 1200 47.7 -> 42.1 (3), 1 x 1600 52.4 -> 48.8
-// (3), 1 x 4096 90 (5; 3 is 4 % slower).
+// (3), 1 x 4096 90 (5; 3 is 4 % slower); at 48 1 x 8192 262 -> 235 and 1 x
+// 16000 536 -> 440 (whole -> 4), at 64 1 x 12000 421 -> 390 (whole -> 3).
 //
 // More sequences: only the device knows their lengths. It weighs its plan against scanning every
 // sequence whole (plan_jobs); what is decided here is whether it may cut, since a pass A without
@@ -41,14 +42,15 @@ int64_t max_chunks(int64_t T, int64_t N) { return (T + kChunkH - 1) / kChunkH + 
 constexpr double kSegOdds = 3.75;
 constexpr double kCallRest = 45.0;  // k cycles of a call besides its chunks (prep, starts)
 
-int seg_count(int64_t T, int64_t N, int64_t HV)
+// (cached: chunk times as if everything stayed in the cache; see prefill_launch)
+int seg_count(int64_t T, int64_t N, int64_t HV, bool cached)
 {
     // (the job planner runs one sequence per lane in the self-planned prep kernel)
     if (T <= 0 || N <= 0 || N > gdn::kSegSeqMax || N * HV * 3 > 256)
         return 1;
     const int64_t cmax = (T + kChunkH - 1) / kChunkH;  // no sequence has more chunks
     const double w = gdn::kSegFirstWeight, h = 0.5 * gdn::kSegChainChunks;
-    const double whole = cmax * gdn::chunk_cost(N * HV);
+    const double whole = cmax * gdn::whole_chunk_cost(N * HV, cached ? 0.f : (float)(cmax * HV));
     // the planner cuts c chunks into at most G*(c) segments, its closed-form optimum (rising with
     // c; +1 for the device's float rounding): capacities sized for that are tight
     const int64_t gs = (int64_t)(1.0 - w + std::sqrt(w * w + w + (double)cmax / h)) + 1;
@@ -78,10 +80,10 @@ struct Layout {
     int64_t jobs, seg_sin, seg_r, seg_mt;
 };
 
-Layout layout(int64_t T, int64_t N, int64_t HV)
+Layout layout(int64_t T, int64_t N, int64_t HV, bool cached)
 {
     Layout L;
-    L.G = seg_count(T, N, HV);
+    L.G = seg_count(T, N, HV, cached);
     L.capA = N * (2 * L.G - 3);
     L.capC = N * (L.G - 1);
     L.nc = max_chunks(T, N);
@@ -144,10 +146,20 @@ extern "C" int64_t gdn_prefill_workspace_size(int32_t total_tokens, int32_t num_
         return gdn_set_error(GDN_EINVAL, "gdn_prefill_workspace_size: bad sizes T=%d N=%d "
                              "HQK=%d HV=%d D=%d", total_tokens, num_seqs, num_qk_heads,
                              num_v_heads, head_size);
-    return layout(total_tokens, num_seqs, num_v_heads).total;
+    return layout(total_tokens, num_seqs, num_v_heads, false).total;
+}
+
+int64_t gdn::prefill_workspace_cached(int64_t T, int64_t N, int64_t HV)
+{
+    return layout(T, N, HV, true).total;
 }
 
 extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
+{
+    return gdn::prefill_launch(p, stream, false);
+}
+
+int gdn::prefill_launch(const gdn_prefill_params *p, void *stream, bool cached)
 {
     gdn_begin_call();
     if (!p || p->struct_size != (int32_t)sizeof(gdn_prefill_params))
@@ -200,7 +212,7 @@ extern "C" int gdn_prefill_launch(const gdn_prefill_params *p, void *stream)
     if (p->A_log_stride < 0 || p->A_log_stride >= kMaxGateStride || p->dt_bias_stride < 0 ||
         p->dt_bias_stride >= kMaxGateStride)
         return gdn_set_error(GDN_ELAYOUT, "gdn_prefill: A_log / dt_bias strides must be in [0, 2^31)");
-    const Layout L = layout(T, N, HV);
+    const Layout L = layout(T, N, HV, cached);
     if (L.nc > 0x7fffffff)
         return gdn_set_error(GDN_EINVAL, "gdn_prefill: too many chunks");
     if (!p->workspace || p->workspace_bytes < L.total || !aligned(p->workspace, 256))

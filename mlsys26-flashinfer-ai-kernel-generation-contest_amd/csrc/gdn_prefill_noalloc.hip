@@ -66,10 +66,15 @@ extern "C" int gdn_prefill_launch_noalloc(const gdn_prefill_params *p, void *str
     gdn_begin_call();
     if (!p || p->struct_size != (int32_t)sizeof(gdn_prefill_params))
         return gdn_set_error(GDN_EINVAL, "gdn_prefill_launch_noalloc: params NULL or struct_size mismatch");
-    const int64_t need = gdn_prefill_workspace_size(p->total_tokens, p->num_seqs, p->num_qk_heads,
-                                                    p->num_v_heads, p->head_size);
+    int64_t need = gdn_prefill_workspace_size(p->total_tokens, p->num_seqs, p->num_qk_heads,
+                                              p->num_v_heads, p->head_size);
     if (need < 0)
         return (int)need;  // message set by gdn_prefill_workspace_size
+    // where only the segments' slots do not fit (one sequence of 43 to 64 v-heads and 6 to 9
+    // thousand tokens), the plan that does without them
+    const bool cached = need > kScratchBytes;
+    if (cached)
+        need = gdn::prefill_workspace_cached(p->total_tokens, p->num_seqs, p->num_v_heads);
     if (need > kScratchBytes)
         return gdn_set_error(GDN_EWORKSPACE,
                              "gdn_prefill_launch_noalloc: T=%d N=%d HV=%d needs %lld bytes of "
@@ -91,5 +96,5 @@ extern "C" int gdn_prefill_launch_noalloc(const gdn_prefill_params *p, void *str
     gdn_prefill_params q = *p;
     q.workspace = ws;
     q.workspace_bytes = kScratchBytes;
-    return gdn_prefill_launch(&q, stream);
+    return gdn::prefill_launch(&q, stream, cached);
 }

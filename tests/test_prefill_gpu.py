@@ -481,6 +481,9 @@ def test_prefill_segments_mixed(dev, lens, hqk, hv, cut):
     # ten of 44-50 chunks: cut in 3 both passes would need 8 waves and lose
     ([3000, 2900, 3100, 2950, 3050, 2800, 3200, 2850, 3150, 2990], 4, 8, (0, 10)),
     (varlen_lengths(8, seed=7), 4, 8, (0, 0)),  # 3-12 chunks: not offered
+    # one sequence at 48 v-heads: whole, and in 4 segments where the call outgrows the cache
+    ([4096], 24, 48, (0, 0)),
+    ([8192], 24, 48, (5, 3)),
 ])
 def test_prefill_segment_planner(dev, lens, hqk, hv, plan):
     """Segment plans on few sequences (mild decay, so every chained state carries into the next

@@ -75,6 +75,33 @@ def test_noalloc_rejects_oversize(dev):
     assert "static scratch" in _lib.last_error()
 
 
+def test_noalloc_without_room_for_segments(dev):
+    """One sequence whose records fit the static scratch but whose segments' slots do not (7000
+    tokens, 44 v-heads): taken with fewer segments, within the parity bars of the plan that the
+    caller-owned workspace gets."""
+    lib = _lib.load()
+    T, hqk, hv = 7000, 22, 44
+    cap = lib.gdn_prefill_noalloc_capacity()
+    assert lib.gdn_prefill_workspace_size(T, 1, hqk, hv, 128) > cap
+    g = prefill_inputs([T], hqk=hqk, hv=hv, seed=11, with_state=True, gates="mild").to(dev)
+    outs = []
+    for fn in (lib.gdn_prefill_launch, lib.gdn_prefill_launch_noalloc):
+        out = torch.full((T, hv, 128), 5.0, dtype=torch.bfloat16, device=dev)
+        ns = torch.full((1, hv, 128, 128), 5.0, dtype=torch.float32, device=dev)
+        P, _, _, copy_back, keep, stream = _prefill_marshal(
+            *g.args(), out, ns, with_workspace=not outs)
+        assert not copy_back
+        print(f"[segments in scratch] {fn.__name__}", flush=True)
+        _lib.check(fn(ctypes.byref(P), ctypes.c_void_p(stream.cuda_stream)), fn.__name__)
+        torch.cuda.synchronize()
+        outs.append((out, ns))
+        del keep
+    (o1, s1), (o2, s2) = outs
+    vo, vs = check_output(o2, o1.float()), check_state(s2, s1)
+    print(f"[segments in scratch] output {vo} | state {vs}", flush=True)
+    assert vo.ok and vs.ok
+
+
 def test_noalloc_in_graph_after_eager_call(dev):
     """After an eager call on the device, a noalloc prefill captured into a HIP graph
     replays bit-identically to the eager result (three replays, eager noalloc calls on
