@@ -140,7 +140,9 @@ int gdn_prefill_launch(const gdn_prefill_params *p, void *stream);
  * (96 MiB) per device, set up on the first call on that device and held until the
  * process ends; p->workspace and p->workspace_bytes are ignored. Sizes whose
  * gdn_prefill_workspace_size exceeds it fail with GDN_EWORKSPACE before any launch
- * (at 32 v-heads: about 11,000 tokens in 16 sequences). Calls on one device share the
+ * (at 32 v-heads: about 11,000 tokens in 16 sequences), except where a plan with fewer
+ * segments fits (one sequence of some 6000 to 9000 tokens at 43 to 64 v-heads), which is
+ * then used. Calls on one device share the
  * array: calls that overlap in time on one device (other streams, unordered host
  * threads) race. Nothing is allocated, freed or memset.
  */

@@ -290,10 +290,12 @@ constexpr int kQueueIdx = 8;  // header[8 .. 15]: next job slot per XCD of the q
 // the longest sequence stays below 0.65 of the load per CU, a (sequence, v-head)'s start and
 // end counted as two chunks. Measured on MI355X over 107 batches of 26 to 500 sequences at 4 to
 // 32 v-heads, 1 to 4 of them long: wide / 8-wave 0.87 to 0.98 up to a ratio of 0.55, 1.04 to
-// 1.13 at 0.9 to 1, 1.2 to 1.3 above 1.3; this line never costs more than 1.1 %. Whole prefills
-// without the choice -> with it: 5000 and 40 of 64 tokens at 32 v-heads 315 -> 253 us, 16384 and
-// 99 of 64 at 8 874 -> 682, 1024 and 30 of 64 at 32 87 -> 74; the launch that finds nothing costs
-// 1.8 us (100 of 64 at 32 155 -> 157).
+// 1.13 at 0.9 to 1, 1.2 to 1.3 above 1.3; this line never costs more than 1.1 %
+// of either. Whole prefills without the choice -> with it: 5000 and 40 of 64 tokens at 32 v-heads
+// 315 -> 252 us, 16384 and 99 of 64 at 8 872 -> 691, 1024 and 30 of 64 at 32 87 -> 74; the launch
+// that finds nothing costs 1.8 us (100 of 64 at 32 154 -> 156). The queue's own cost (up to 5 %
+// against one workgroup per job) leaves the line where it is: over 170 more batches every ratio
+// from 0.5 to 0.65 gives the same mean.
 __device__ inline void choose_wide(const PlanArgs &p, float cmax, float total)
 {
     const float load = (total + 2.f * (float)p.N) * (float)p.HO / (float)p.wide_cus;
